@@ -27,13 +27,21 @@
 // that XCD's L2.
 #include "fft_lds.h"
 #include "lsd_internal.h"
+#include "physwave.h"
 
 namespace lsd {
 
-// Threads per workgroup: one per phi point, 512 for Ph <= 512 and 1024 up
-// to Ph = 1024.
+// Threads per workgroup: one per phi point, the least of 64, 128, 256, 512
+// and 1024 that is not below Ph: idle waves still meet every barrier (FP64,
+// 64 shells of 96 x 48: 197 us per launch with 512 threads, 41 us with 64;
+// 32 shells of 48 x 96: 55 us with 512, 25 us with 128).
 constexpr int PF_THREADS = 512;
 constexpr int PF_THREADS_MAX = 1024;
+static int pf_threads(int Ph) {
+    int nt = 64;
+    while (nt < Ph && nt < PF_THREADS_MAX) nt *= 2;
+    return nt;
+}
 constexpr int PF_EPT = 8;      // 8 sequences x 512 points = one radix-8 butterfly per thread
 constexpr int PF_MAXSEQ = 8;
 
@@ -565,8 +573,38 @@ __global__ void __launch_bounds__(NT) k_physfuse(PhysArgs<R> a) {
 }
 
 bool physfuse_supported(const Ctx& c) {
-    const int nt = c.Ph <= PF_THREADS ? PF_THREADS : PF_THREADS_MAX;
-    return c.Ph <= PF_THREADS_MAX && c.Th % 2 == 0 && 6 * c.M <= PF_ITEMS * nt;
+    return c.Ph <= PF_THREADS_MAX && c.Th % 2 == 0 && 6 * c.M <= PF_ITEMS * pf_threads(c.Ph);
+}
+
+// The wave form (physwave.h); 1: a length it is not instantiated for.
+static int physwave_launch(Ctx& c, const PhysArgs<float>& a) {
+    PwArgs<float> w;
+    w.N = a.N;
+    w.Th = a.Th;
+    w.Th2 = a.Th2;
+    w.M = a.M;
+    w.MP = a.MP;
+    w.cor = a.cor;
+    w.cmag = a.cmag;
+    w.qc = a.qc;
+    w.qx = a.qx;
+    w.scale = a.scale;
+    w.cod = a.cod;
+    w.comp = a.comp;
+    w.mag = a.mag;
+    w.gp = a.gp;
+    w.sn = a.sn;
+    w.fourier = a.fourier;
+    w.folded = a.folded;
+    w.tw = a.tw;
+    w.cfl = a.cfl;
+    w.cfl_d = a.cfl_d;
+    w.ep = a.ep;
+    w.eE = a.eE;
+    w.ePm = a.ePm;
+    int rc = physwave_f32_small(c, w, c.cfl_on);
+    if (rc > 0) rc = physwave_f32_large(c, w, c.cfl_on);
+    return rc > 0 ? physwave_f32_long(c, w, c.cfl_on) : rc;
 }
 
 template <typename R>
@@ -604,6 +642,21 @@ static int physfuse_launch(Ctx& c, const void* fourier, void* folded, const void
     a.eE = (R)k.E;
     a.ePm = (R)k.Pm;
     if (c.cfl_on) c.cfl_parts = c.Th2;
+    // FP32 takes the wave form at the lengths it is instantiated for, where
+    // the 3/2 rule leaves the upper third of the orders empty.  FP64 keeps
+    // this form and its rounding: plain runs go on bit for bit from recorded
+    // states (the wave form in FP64 measured 31 against 55 us at 48 x 96, 32
+    // shells and 535 against 640 us at 256 x 512, 96 shells, but chaotic runs
+    // leave their recorded trajectories with any other order of the sums).
+    // Mixed runs that time-step the inner core's rotation keep it too: their
+    // viscous torque is a wall gradient that carries the banded solves'
+    // roundoff, amplified by 1/dt at the start-up steps of 1e-8.
+    if constexpr (sizeof(R) == 4) {
+        if (3 * c.M <= c.Ph && !c.cfg.rot) {
+            const int rc = physwave_launch(c, a);
+            if (rc <= 0) return rc;
+        }
+    }
     const int nblk = ((a.ngroups + 7) / 8) * 8 * PF_GROUP<R>;
     const bool r512 = physfuse_r512(c.Ph);
     const size_t lds = physfuse_lds<V>(c.Ph, r512);
@@ -614,25 +667,30 @@ static int physfuse_launch(Ctx& c, const void* fourier, void* folded, const void
                  (double)sizeof(V) * c.N * c.M * ((double)nin * c.Th + (double)nout * 2 * c.Th2));
     const bool pruned = r512 && c.M > 128 && c.M <= 192;
     const dim3 g(nblk);
-    if (c.cfl_on) {
-        if (pruned) hipLaunchKernelGGL((k_physfuse<R, true, PF_THREADS, true, true>), g, dim3(PF_THREADS), lds, c.stream, a);
-        else if (r512)
-            hipLaunchKernelGGL((k_physfuse<R, true, PF_THREADS, true, false>), g, dim3(PF_THREADS), lds, c.stream, a);
-        else if (c.Ph <= PF_THREADS)
-            hipLaunchKernelGGL((k_physfuse<R, false, PF_THREADS, true, false>), g, dim3(PF_THREADS), lds, c.stream, a);
-        else
-            hipLaunchKernelGGL((k_physfuse<R, false, PF_THREADS_MAX, true, false>), g, dim3(PF_THREADS_MAX), lds,
-                               c.stream, a);
-    } else if (pruned) {
-        hipLaunchKernelGGL((k_physfuse<R, true, PF_THREADS, false, true>), g, dim3(PF_THREADS), lds, c.stream, a);
+#define PF_RUN(R512, NT, CFL, PRUNED) \
+    hipLaunchKernelGGL((k_physfuse<R, R512, NT, CFL, PRUNED>), g, dim3(NT), lds, c.stream, a)
+#define PF_RUN_NT(NT)                              \
+    do {                                           \
+        if (c.cfl_on) PF_RUN(false, NT, true, false); \
+        else PF_RUN(false, NT, false, false);      \
+    } while (0)
+    if (pruned) {
+        if (c.cfl_on) PF_RUN(true, PF_THREADS, true, true);
+        else PF_RUN(true, PF_THREADS, false, true);
     } else if (r512) {
-        hipLaunchKernelGGL((k_physfuse<R, true, PF_THREADS, false, false>), g, dim3(PF_THREADS), lds, c.stream, a);
-    } else if (c.Ph <= PF_THREADS) {
-        hipLaunchKernelGGL((k_physfuse<R, false, PF_THREADS, false, false>), g, dim3(PF_THREADS), lds, c.stream, a);
+        if (c.cfl_on) PF_RUN(true, PF_THREADS, true, false);
+        else PF_RUN(true, PF_THREADS, false, false);
     } else {
-        hipLaunchKernelGGL((k_physfuse<R, false, PF_THREADS_MAX, false, false>), g, dim3(PF_THREADS_MAX), lds,
-                           c.stream, a);
+        switch (pf_threads(c.Ph)) {
+        case 64: PF_RUN_NT(64); break;
+        case 128: PF_RUN_NT(128); break;
+        case 256: PF_RUN_NT(256); break;
+        case 512: PF_RUN_NT(512); break;
+        default: PF_RUN_NT(1024); break;
+        }
     }
+#undef PF_RUN_NT
+#undef PF_RUN
     LSD_HIP(hipGetLastError());
     return LSD_OK;
 }
