@@ -1,0 +1,43 @@
+"""The network's fused passes at the edges of their tiles (rows around the 32
+of a workgroup and the 128 and 512 of the gradient chunks, widths that fill
+64, 128 or 256 columns partly, inputs with unaligned rows, many outputs) and
+the GEMM-per-layer form past 256 inputs, against the CPU oracle with the
+bounds of test_gpu_mlp.py (outputs and gradients 2e-3 in relative L2: BF16
+operands, sums in another order)."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+from lsd.gpu import Mlp
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
+import mlp_ref  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n_in,width,n_out,rows", [
+    (92, 256, 10, 1), (92, 256, 10, 33), (92, 256, 10, 513), (92, 250, 10, 129), (17, 48, 3, 640), (93, 200, 33, 127),
+    (92, 128, 10, 1025), (256, 256, 256, 96), (92, 64, 64, 31), (1, 16, 1, 512), (300, 256, 10, 200), (92, 260, 10, 65)])
+def test_sizes(n_in, width, n_out, rows):
+    rng = np.random.default_rng(rows + width)
+    m = Mlp(n_in, width, n_out, seed=3)
+    p = m.params()
+    X = rng.standard_normal((rows, n_in)).astype(np.float32)
+    T = rng.standard_normal((rows, n_out)).astype(np.float32)
+    y = m.forward(X)
+    yo, _ = mlp_ref.forward(p, X, n_in, width, n_out, rb=True)
+    assert np.linalg.norm(y - yo) <= 2e-3 * np.linalg.norm(yo)
+    loss, g = m.grad(X, T)
+    lo, go = mlp_ref.loss_and_grad(p, X, T, n_in, width, n_out, rb=True)
+    assert abs(loss - lo) <= 1e-3 * lo
+    assert np.linalg.norm(g - go) <= 2e-3 * np.linalg.norm(go)
+    # a step of training on a batch that leaves a short rest: the losses are
+    # those of the batches
+    batch = max(1, 2 * rows // 3)
+    losses = m.train(X, T, batch, 2, 0.0)
+    part = [m.grad(X[:batch], T[:batch])[0], m.grad(X[batch:], T[batch:])[0] if rows > batch else m.grad(X, T)[0]]
+    assert np.array_equal(losses, np.array(part, dtype=np.float32))
+    m.close()
