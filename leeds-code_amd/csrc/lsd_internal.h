@@ -342,6 +342,8 @@ int launch_vec_prep(Ctx& c, int nf, const double2* const* T, const double2* cons
                     bool f32);
 int launch_scal_prep(Ctx& c, int nf, const double2* const* C, void* const* dC, void* const* Cc, bool f32);
 int launch_spec_post(Ctx& c, bool f32);
+int launch_split_coll(Ctx& c, const double2* in, double* re, double* im);
+int launch_merge_coll(Ctx& c, const double* re, const double* im, double2* out);
 int launch_layout_spec2coll(Ctx& c, const double* re, const double* im, double2* out);
 int launch_layout_coll2spec(Ctx& c, const double2* in, double* re, double* im);
 

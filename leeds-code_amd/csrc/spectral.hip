@@ -287,6 +287,21 @@ __global__ void k_coll2spec(int H, int N, const double2* __restrict__ in, double
     im[idx] = v.y;
 }
 
+// coll double2 [h][n] to and from its Re and Im arrays (the host's coll layout).
+__global__ void k_split_coll(size_t n, const double2* __restrict__ in, double* __restrict__ re,
+                             double* __restrict__ im) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double2 v = in[i];
+    re[i] = v.x;
+    im[i] = v.y;
+}
+__global__ void k_merge_coll(size_t n, const double* __restrict__ re, const double* __restrict__ im,
+                             double2* __restrict__ out) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) out[i] = make_double2(re[i], im[i]);
+}
+
 static dim3 grid1(size_t n) { return dim3((unsigned)((n + 255) / 256)); }
 
 // Column-blocked launch shape of the spectral kernels, and their LDS
@@ -381,6 +396,20 @@ int launch_spec_post(Ctx& c, bool f32) {
                            c.L, c.d_hl, c.d_r, c.d_r1dr, c.d_ll, pp, c.d_spec_out, c.d_f[LSD_COD], c.d_f[LSD_COMP],
                            c.d_f[LSD_N_VEL_TOR], c.d_f[LSD_N_VEL_POL], c.d_f[LSD_N_COD], c.d_f[LSD_N_COMP],
                            c.d_f[LSD_N_MAG_TOR], c.d_f[LSD_N_MAG_POL]);
+    LSD_HIP(hipGetLastError());
+    return LSD_OK;
+}
+
+int launch_split_coll(Ctx& c, const double2* in, double* re, double* im) {
+    const size_t n = c.coll_elems();
+    hipLaunchKernelGGL(k_split_coll, grid1(n), dim3(256), 0, c.stream, n, in, re, im);
+    LSD_HIP(hipGetLastError());
+    return LSD_OK;
+}
+
+int launch_merge_coll(Ctx& c, const double* re, const double* im, double2* out) {
+    const size_t n = c.coll_elems();
+    hipLaunchKernelGGL(k_merge_coll, grid1(n), dim3(256), 0, c.stream, n, re, im, out);
     LSD_HIP(hipGetLastError());
     return LSD_OK;
 }
