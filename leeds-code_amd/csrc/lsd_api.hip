@@ -291,7 +291,8 @@ static int create(const lsd_config* cfg, int device, Ctx** out) {
     for (int k = 0; k < 6; k++)
         if (dalloc(&c->d_hist[k], HN)) return LSD_E_HIP;
     const bool direct = solve_direct_supported(N);
-    if (direct) {
+    c->solve_padded = c->mixed && !direct && N <= SOLVE_DIRECT_MAX_N;
+    if (direct || c->solve_padded) {
         for (int k = 0; k < 6; k++)
             if (dalloc(&c->d_rhs[k], HN)) return LSD_E_HIP;
         if (dalloc(&c->d_rhs2, HN)) return LSD_E_HIP;
@@ -302,7 +303,7 @@ static int create(const lsd_config* cfg, int device, Ctx** out) {
     c->solve_direct_ok = direct;
     c->hb_form[0] = 32;
     c->hb_form[1] = solve_block_harmonics(N, c->mixed);
-    c->hb_form[2] = c->mixed ? solve_block_harmonics(N, false) : 0;
+    c->hb_form[2] = c->solve_padded ? 32 : c->mixed ? solve_block_harmonics(N, false) : 0;
     if (c->hb_form[1] < 1 && !direct) {
         set_error("N too large for the banded-solve kernels");
         return LSD_E_CONFIG;

@@ -199,9 +199,10 @@ struct Ctx {
     int var[LSD_V_COUNT] = {4, 8, 8, 0, 0};
     bool ana_wide_ok = false;          // the wide-load FP32 analysis applies (even Th2)
     bool solve_direct_ok = false;      // the two-pass solves apply (N in {32, 48, 64, 96})
+    bool solve_padded = false;         // mixed forms, other N <= 128: they run variant 2 on padded columns
     // solve blocks of the two forms: [0] two-pass (32 harmonics), [1] LDS-column
     // solve block sets: 0 two-pass, 1 LDS-column, 2 LDS-column with FP64
-    // factors in the mixed forms
+    // factors in the mixed forms (solve_padded: register columns, 32)
     int4* d_sblk[3] = {nullptr, nullptr, nullptr};
     int* d_sord[3] = {nullptr, nullptr, nullptr};
     int nblk_form[3] = {0, 0, 0};
@@ -400,6 +401,7 @@ double corrector_norms(const Ctx& c);
 
 // solve_direct.hip
 bool solve_direct_supported(int N);
+constexpr int SOLVE_DIRECT_MAX_N = 128;  // rows of the longest register column
 int launch_solve_direct(Ctx& c, bool pred);
 
 }  // namespace lsd

@@ -1,5 +1,11 @@
-// Predictor / corrector solves for the radial resolutions the library is
-// built for (N fixed at compile time).
+// Predictor / corrector solves with the column in registers: N in {32, 48,
+// 64, 96} at compile time, and in the mixed forms any N <= 128 in a column
+// padded with identity rows to a multiple of 16 (plain runs of other N keep
+// the LDS-column kernels and their rounding).  At L = M = 256, N = 128 the
+// mixed form's solves go from 2485 (predictor) and 2230 us (corrector) with
+// the LDS-column kernels, whose LDS holds 20 harmonics a wave and two waves a
+// CU, to 297 + 297 and 530 us, within a factor 1.25 of their memory traffic
+// at the rate of a large copy.
 //
 // One 64-lane wave per block of up to 32 harmonics of one degree l (lane =
 // harmonic, Re/Im part), so every lane needs the same factors, which are
@@ -138,7 +144,7 @@ __device__ __forceinline__ double2 band_acc(double2 acc, const double* __restric
 // degree l) and field: the Y band of (field, l) and the block's state
 // columns are staged in LDS, so each point's 7-term band row reads LDS only.
 constexpr int RHS_BLK = 1024;
-constexpr int RHS_IT = (32 * 96 + RHS_BLK - 1) / RHS_BLK;  // points per thread at 32 harmonics, N <= 96
+constexpr int RHS_IT = (32 * SOLVE_DIRECT_MAX_N + RHS_BLK - 1) / RHS_BLK;  // points per thread at 32 harmonics
 
 template <bool H32>
 __global__ void __launch_bounds__(RHS_BLK) k_rhs_pred(DirArgs a, float inv_n) {
@@ -227,7 +233,7 @@ constexpr int SWEEP_AHEAD = 2;  // rows of factors read from LDS ahead of the sw
 // LDS or division latency sits on the serial chain.
 template <int N, typename T>
 __device__ __forceinline__ void gbtrs_reg(T (&b)[N], const T* ab, const T* rd, const unsigned* __restrict__ pk) {
-    constexpr int NPK = (N + 15) / 16;
+    constexpr int NPK = (N + 15) / 16;  // also that of a padded column: it ends in the last word's rows
     unsigned pw[NPK];
 #pragma unroll
     for (int k = 0; k < NPK; k++) pw[k] = pk[k];
@@ -289,23 +295,42 @@ struct DirSmem {
 
 // Copies the factors of (kind, l) into LDS, with the reciprocal diagonal.
 // Callers synchronise before the data are read and before they are replaced.
-template <int N>
+// Padded columns (EXACT false: n < N rows) continue with rows of the
+// identity, and the multipliers that would reach them are zero, so the rows
+// of the band get the results of a sweep over n rows.
+template <int N, bool EXACT>
 __device__ __forceinline__ void stage_factors(const DirArgs& a, DirSmem<N>& s, int kind, int l) {
-    const double* src = a.lu + ((size_t)kind * a.L + l) * N * LSD_LDAB;
+    const int n = EXACT ? N : a.N;
+    const double* src = a.lu + ((size_t)kind * a.L + l) * n * LSD_LDAB;
     constexpr int NA = (N * LSD_LDAB + 63) / 64;
     double v[NA];
 #pragma unroll
     for (int k = 0; k < NA; k++) {
         const int i = threadIdx.x + 64 * k;
-        if (i < N * LSD_LDAB) v[k] = src[i];
+        if (i < N * LSD_LDAB) v[k] = src[EXACT ? i : min(i, n * LSD_LDAB - 1)];
     }
 #pragma unroll
     for (int k = 0; k < NA; k++) {
         const int i = threadIdx.x + 64 * k;
         if (i < N * LSD_LDAB) {
+            if constexpr (!EXACT) {
+                const int j = i / LSD_LDAB, r = i % LSD_LDAB;
+                if (j >= n) v[k] = r == 2 * LSD_KL ? 1.0 : 0.0;
+                else if (r > 2 * LSD_KL && j + r - 2 * LSD_KL >= n) v[k] = 0.0;
+            }
             s.ab[i] = v[k];
             if (i % LSD_LDAB == 2 * LSD_KL) s.rd[i / LSD_LDAB] = 1.0 / v[k];
         }
+    }
+}
+
+// The Green's functions of degree l (zero in padded rows).
+template <int N, bool EXACT>
+__device__ __forceinline__ void stage_green(const DirArgs& a, DirSmem<N>& s, int l) {
+    const int n = EXACT ? N : a.N;
+    for (int i = threadIdx.x; i < 2 * N; i += 64) {
+        const int k = i / N, r = i - k * N;
+        s.g[i] = (EXACT || r < n) ? a.gre[(size_t)l * 2 * n + k * n + r] : 0.0;
     }
 }
 
@@ -319,14 +344,55 @@ __device__ __forceinline__ const unsigned* pivots(const DirArgs& a, int kind, in
 // VGPRs of two waves per SIMD at N = 96.
 constexpr int DIR_BATCH = 16;
 
-// Predictor solves: x* = X^-1 b for the right-hand sides of k_rhs_pred.  At
-// most 256 VGPRs, so two waves share each SIMD.
-template <int N>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_spred(DirArgs a) {
+// Columns of n rows in N registers: all of them (EXACT), or N rounded up to a
+// batch, whose last rows are identity rows (see stage_factors).  The padding
+// ends within the last batch, so only its rows compare with n.
+template <int N, bool EXACT>
+struct ColRows {
+    int n;
+    __device__ __forceinline__ explicit ColRows(int rows) : n(EXACT ? N : rows) {}
+    static constexpr int TAIL = N - DIR_BATCH;
+    // row r holds a value of the column / is its last row
+    __device__ __forceinline__ bool in(int r) const { return EXACT || r < TAIL || r < n; }
+    __device__ __forceinline__ bool last(int r) const { return EXACT ? r == N - 1 : r >= TAIL && r == n - 1; }
+    __device__ __forceinline__ int clamp(int r) const { return EXACT || r < TAIL ? r : min(r, n - 1); }
+    __device__ __forceinline__ double end(const double (&b)[N]) const {
+        if constexpr (EXACT) return b[N - 1];
+        // pinned copies: a plain select would be merged into one access by
+        // index, which puts the column in scratch memory
+        double v = b[TAIL];
+#pragma unroll
+        for (int r = TAIL + 1; r < N; r++) {
+            double w = b[r];
+            pin(w);
+            v = r == n - 1 ? w : v;
+        }
+        return v;
+    }
+};
+template <bool EXACT, int N, typename C>
+__device__ __forceinline__ void load_rows(const ColRows<N, EXACT>& cr, const C* col, int n, int part, double& v0,
+                                          double& v1) {
+    if constexpr (EXACT) {
+        load_pair(col, n, part, v0, v1);
+    } else {
+        // the row of this lane, clamped; load_pair reads col[n + part]
+        const int r = cr.clamp(n + part);
+        load_pair(col + (r - n - part), n, part, v0, v1);
+    }
+}
+
+// Predictor solves: x* = X^-1 b for the right-hand sides of k_rhs_pred.  Up
+// to N = 96 at most 256 VGPRs, so two waves share each SIMD; longer columns
+// have a SIMD to themselves.
+template <int N, bool EXACT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(N <= 96 ? 2 : 1))) k_spred(DirArgs a) {
     static_assert(N % DIR_BATCH == 0, "N must be a multiple of the batch");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     DirSmem<N>& s = *reinterpret_cast<DirSmem<N>*>(smem_raw);
     constexpr int BT = DIR_BATCH;
+    const ColRows<N, EXACT> cr(a.N);
+    const int NR = cr.n;  // rows of a column
     const int f = blockIdx.y;
     const int t = threadIdx.x;
     if (a.on[f]) {
@@ -340,42 +406,47 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
         // ahead of the factor staging so both are in flight together
         // (8-byte loads into the column: pair loads would hold 16 bytes per
         // row until every row has arrived)
-        const double* src = reinterpret_cast<const double*>(pick(a.rhs, f) + (size_t)h * N) + part;
+        const double* src = reinterpret_cast<const double*>(pick(a.rhs, f) + (size_t)h * NR) + part;
         double b[N];
 #pragma unroll
-        for (int n = 0; n < N; n++) b[n] = src[2 * n];
+        for (int n = 0; n < N; n++) b[n] = src[2 * cr.clamp(n)];
+        if constexpr (!EXACT) {
+#pragma unroll
+            for (int n = cr.TAIL; n < N; n++) b[n] = cr.in(n) ? b[n] : 0.0;
+        }
         if (solve) {
-            stage_factors<N>(a, s, lu_kind(f), l);
+            stage_factors<N, EXACT>(a, s, lu_kind(f), l);
             if (f == 1)
-                for (int i = t; i < 2 * N; i += 64) s.g[i] = a.gre[(size_t)l * 2 * N + i];
+                stage_green<N, EXACT>(a, s, l);
         }
         __syncthreads();
         if (solve) gbtrs_reg<N, double>(b, s.ab, s.rd, pivots(a, lu_kind(f), l));
-        double2* xcol = pick(a.x, f) + (size_t)h * N;
+        double2* xcol = pick(a.x, f) + (size_t)h * NR;
         if (f == 1 && solve) {
             // XPol right-hand side: XGre^-1 N + Y x inside, zero on the
             // boundary rows (where the second part is zero)
-            const double2* r2col = a.rhs2 + (size_t)h * N;
+            const double2* r2col = a.rhs2 + (size_t)h * NR;
 #pragma unroll
             for (int c = 0; c < N / BT; c++) {
                 double r2[BT];
 #pragma unroll
-                for (int r = 0; r < BT; r += 2) load_pair(r2col, c * BT + r, part, r2[r], r2[r + 1]);
+                for (int r = 0; r < BT; r += 2) load_rows<EXACT>(cr, r2col, c * BT + r, part, r2[r], r2[r + 1]);
 #pragma unroll
                 for (int r = 0; r < BT; r++) {
                     const int n = c * BT + r;
-                    b[n] = (n == 0 || n == N - 1) ? r2[r] : b[n] + r2[r];
+                    b[n] = (n == 0 || cr.last(n)) ? r2[r] : b[n] + r2[r];
+                    b[n] = cr.in(n) ? b[n] : 0.0;
                     pin(b[n]);
                 }
                 BATCH_FENCE();
             }
             __syncthreads();
-            stage_factors<N>(a, s, 1, l);
+            stage_factors<N, EXACT>(a, s, 1, l);
             __syncthreads();
             gbtrs_reg<N, double>(b, s.ab, s.rd, pivots(a, 1, l));
             // vel_gre_adjust (velocity.F90:445-465) on x*
             const double* ig = a.invg + l * 4;
-            const double bi = b[0], bo = b[N - 1];
+            const double bi = b[0], bo = cr.end(b);
             const double ca = ig[0] * bi + ig[2] * bo;
             const double cb = ig[1] * bi + ig[3] * bo;
 #pragma unroll
@@ -384,13 +455,13 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
                 for (int r = 0; r < BT; r += 2) {
                     const int n = c * BT + r;
                     store_pair(xcol, n, part, b[n] - ca * s.g[n] - cb * s.g[N + n],
-                               b[n + 1] - ca * s.g[n + 1] - cb * s.g[N + n + 1], act);
+                               b[n + 1] - ca * s.g[n + 1] - cb * s.g[N + n + 1], act && cr.in(n + part));
                 }
                 BATCH_FENCE();
             }
         } else {
 #pragma unroll
-            for (int n = 0; n < N; n += 2) store_pair(xcol, n, part, b[n], b[n + 1], act);
+            for (int n = 0; n < N; n += 2) store_pair(xcol, n, part, b[n], b[n + 1], act && cr.in(n + part));
         }
     }
 }
@@ -398,13 +469,15 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
 // Corrector: b = c (N* - N) formed in registers (N* in the column, the saved
 // N streamed and replaced), x += X^-1 b, with the tim_addcorr norms; one
 // wave per (solve block, field).
-template <int N, bool H32>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_scorr(DirArgs a) {
+template <int N, bool H32, bool EXACT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(N <= 96 ? 2 : 1))) k_scorr(DirArgs a) {
     static_assert(N % DIR_BATCH == 0, "N must be a multiple of the batch");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ double red[2][64];
     DirSmem<N>& s = *reinterpret_cast<DirSmem<N>*>(smem_raw);
     constexpr int BT = DIR_BATCH;
+    const ColRows<N, EXACT> cr(a.N);
+    const int NR = cr.n;  // rows of a column
     const int f = blockIdx.y;
     const int t = threadIdx.x;
     double e2 = 0.0, eic = 0.0;
@@ -417,19 +490,19 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
         // X is solved except for the l = 0 modes of the velocity and the
         // magnetic field
         const bool solve = f == 2 || f == 3 || l != 0;
-        double2* xcol = pick(a.x, f) + (size_t)h * N;
-        const double2* ncol = pick(a.nn, f) + (size_t)h * N;
-        HistT<H32>* hcol = reinterpret_cast<HistT<H32>*>(pick(a.hist, f)) + (size_t)h * N;
+        double2* xcol = pick(a.x, f) + (size_t)h * NR;
+        const double2* ncol = pick(a.nn, f) + (size_t)h * NR;
+        HistT<H32>* hcol = reinterpret_cast<HistT<H32>*>(pick(a.hist, f)) + (size_t)h * NR;
         // N*, every row at once, issued ahead of the factor staging (8-byte
         // loads into the column; the streamed columns below move by pairs)
         const double* nsrc = reinterpret_cast<const double*>(ncol) + part;
         double b[N];
 #pragma unroll
-        for (int n = 0; n < N; n++) b[n] = nsrc[2 * n];
+        for (int n = 0; n < N; n++) b[n] = nsrc[2 * cr.clamp(n)];
         if (solve) {
-            stage_factors<N>(a, s, lu_kind(f), l);
+            stage_factors<N, EXACT>(a, s, lu_kind(f), l);
             if (f == 1)
-                for (int i = t; i < 2 * N; i += 64) s.g[i] = a.gre[(size_t)l * 2 * N + i];
+                stage_green<N, EXACT>(a, s, l);
         }
         __syncthreads();
         // b = c (N* - N) inside, zero on the boundary rows; N* saved
@@ -438,14 +511,16 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
         for (int c = 0; c < N / BT; c++) {
             double hv[BT];
 #pragma unroll
-            for (int r = 0; r < BT; r += 2) load_pair(hcol, c * BT + r, part, hv[r], hv[r + 1]);
+            for (int r = 0; r < BT; r += 2) load_rows<EXACT>(cr, hcol, c * BT + r, part, hv[r], hv[r + 1]);
 #pragma unroll
-            for (int r = 0; r < BT; r += 2) store_pair(hcol, c * BT + r, part, b[c * BT + r], b[c * BT + r + 1], act);
+            for (int r = 0; r < BT; r += 2)
+                store_pair(hcol, c * BT + r, part, b[c * BT + r], b[c * BT + r + 1], act && cr.in(c * BT + r + part));
 #pragma unroll
             for (int r = 0; r < BT; r++) {
                 const int n = c * BT + r;
-                const double keep = (n == 0 || n == N - 1) ? 0.0 : 1.0;
+                const double keep = (n == 0 || cr.last(n)) ? 0.0 : 1.0;
                 b[n] = keep * (cimp * (b[n] - hv[r]));
+                b[n] = cr.in(n) ? b[n] : 0.0;
                 pin(b[n]);
             }
             BATCH_FENCE();
@@ -456,14 +531,16 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
         if (solve) gbtrs_reg<N, double>(b, s.ab, s.rd, pivots(a, lu_kind(f), l));
         if (f == 1 && solve) {
             b[0] = 0.0;
-            b[N - 1] = 0.0;
+#pragma unroll
+            for (int n = cr.TAIL; n < N; n++)
+                b[n] = cr.last(n) ? 0.0 : b[n];
             __syncthreads();
-            stage_factors<N>(a, s, 1, l);
+            stage_factors<N, EXACT>(a, s, 1, l);
             __syncthreads();
             gbtrs_reg<N, double>(b, s.ab, s.rd, pivots(a, 1, l));
             // vel_gre_adjust (velocity.F90:445-465) on the correction
             const double* ig = a.invg + l * 4;
-            const double bi = b[0], bo = b[N - 1];
+            const double bi = b[0], bo = cr.end(b);
             const double ca = ig[0] * bi + ig[2] * bo;
             const double cb = ig[1] * bi + ig[3] * bo;
 #pragma unroll
@@ -471,12 +548,12 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
                 double xo[BT];
                 double* xs = reinterpret_cast<double*>(xcol) + part;
 #pragma unroll
-                for (int r = 0; r < BT; r++) xo[r] = xs[2 * (c * BT + r)];
+                for (int r = 0; r < BT; r++) xo[r] = xs[2 * cr.clamp(c * BT + r)];
 #pragma unroll
                 for (int r = 0; r < BT; r++) {
                     const int n = c * BT + r;
                     const double d = b[n] - ca * s.g[n] - cb * s.g[N + n];
-                    if (act) {
+                    if (act && cr.in(n)) {
                         xs[2 * n] = xo[r] + d;
                         e2 = e2 + d * d;
                     }
@@ -490,7 +567,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
                 double xo[BT];
                 double* xs = reinterpret_cast<double*>(xcol) + part;
 #pragma unroll
-                for (int r = 0; r < BT; r++) xo[r] = xs[2 * (c * BT + r)];
+                for (int r = 0; r < BT; r++) xo[r] = xs[2 * cr.clamp(c * BT + r)];
 #pragma unroll
                 for (int r = 0; r < BT; r++) {
                     const int n = c * BT + r;
@@ -502,7 +579,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_
                     }
                 }
 #pragma unroll
-                for (int r = 0; r < BT; r += 2) store_pair(xcol, c * BT + r, part, xo[r], xo[r + 1], act);
+                for (int r = 0; r < BT; r += 2)
+                    store_pair(xcol, c * BT + r, part, xo[r], xo[r + 1], act && cr.in(c * BT + r + part));
                 BATCH_FENCE();
             }
         }
@@ -562,22 +640,42 @@ static DirArgs dir_args(Ctx& c) {
     return a;
 }
 
-template <int N, bool PRED>
+template <int N, bool PRED, bool EXACT>
 static void launch_sdir(Ctx& c, const DirArgs& a) {
     const dim3 grid(c.n_partial_blocks, 6);
-    if (PRED) hipLaunchKernelGGL(k_spred<N>, grid, dim3(64), sizeof(DirSmem<N>), c.stream, a);
-    else if (c.mixed) hipLaunchKernelGGL((k_scorr<N, true>), grid, dim3(64), sizeof(DirSmem<N>), c.stream, a);
-    else hipLaunchKernelGGL((k_scorr<N, false>), grid, dim3(64), sizeof(DirSmem<N>), c.stream, a);
+    const size_t lds = sizeof(DirSmem<N>);
+    if (PRED) hipLaunchKernelGGL((k_spred<N, EXACT>), grid, dim3(64), lds, c.stream, a);
+    else if (EXACT && c.mixed) hipLaunchKernelGGL((k_scorr<N, EXACT, EXACT>), grid, dim3(64), lds, c.stream, a);
+    else hipLaunchKernelGGL((k_scorr<N, false, EXACT>), grid, dim3(64), lds, c.stream, a);
 }
 
+// Compile-time columns where the saved N is FP32 too; every other N of the
+// mixed forms in the next multiple of 16, whose unused rows cost registers
+// and at most 15 rows of the sweeps.  One length per 16 rows instead of 128
+// for all: N = 33 would carry four times its rows, and only N > 96 needs the
+// registers of a whole SIMD.
 template <bool PRED>
 static int launch_sdir_n(Ctx& c, const DirArgs& a) {
-    switch (c.N) {
-    case 32: launch_sdir<32, PRED>(c, a); break;
-    case 48: launch_sdir<48, PRED>(c, a); break;
-    case 64: launch_sdir<64, PRED>(c, a); break;
-    case 96: launch_sdir<96, PRED>(c, a); break;
-    default: set_error("no two-pass solve kernel for this N"); return LSD_E_CONFIG;
+    if (c.solve_direct_ok) {
+        switch (c.N) {
+        case 32: launch_sdir<32, PRED, true>(c, a); break;
+        case 48: launch_sdir<48, PRED, true>(c, a); break;
+        case 64: launch_sdir<64, PRED, true>(c, a); break;
+        case 96: launch_sdir<96, PRED, true>(c, a); break;
+        default: set_error("no two-pass solve kernel for this N"); return LSD_E_CONFIG;
+        }
+    } else {
+        switch ((c.N + DIR_BATCH - 1) / DIR_BATCH) {
+        case 1: launch_sdir<16, PRED, false>(c, a); break;
+        case 2: launch_sdir<32, PRED, false>(c, a); break;
+        case 3: launch_sdir<48, PRED, false>(c, a); break;
+        case 4: launch_sdir<64, PRED, false>(c, a); break;
+        case 5: launch_sdir<80, PRED, false>(c, a); break;
+        case 6: launch_sdir<96, PRED, false>(c, a); break;
+        case 7: launch_sdir<112, PRED, false>(c, a); break;
+        case 8: launch_sdir<128, PRED, false>(c, a); break;
+        default: set_error("no two-pass solve kernel for this N"); return LSD_E_CONFIG;
+        }
     }
     LSD_HIP(hipGetLastError());
     return LSD_OK;
@@ -592,12 +690,13 @@ int launch_solve_direct(Ctx& c, bool pred) {
     const DirArgs a = dir_args(c);
     const int nf = 2 + (c.cfg.cod ? 1 : 0) + (c.cfg.comp ? 1 : 0) + (c.cfg.mag && !c.ic() ? 2 : 0);
     // bytes per element and field: predictor 64 + 32 (48 + 8 + 32 with the
-    // FP32 saved N of the mixed forms), corrector 80 (64)
-    const double per = pred ? (c.mixed ? 88.0 : 96.0) : (c.mixed ? 64.0 : 80.0);
+    // FP32 saved N of the mixed forms at the N of this file), corrector 80 (64)
+    const bool h32 = c.mixed && c.solve_direct_ok;  // FP32 saved N
+    const double per = pred ? (h32 ? 88.0 : 96.0) : (h32 ? 64.0 : 80.0);
     ProfScope ps(c, LSD_K_SOLVE, per * c.coll_elems() * nf);
     if (pred) {
         const size_t lds = sizeof(double2) * (size_t)c.solve_hb * c.N + sizeof(double) * 7 * (size_t)c.N;
-        if (c.mixed)
+        if (h32)
             hipLaunchKernelGGL(k_rhs_pred<true>, dim3(c.n_partial_blocks, 6), dim3(RHS_BLK), lds, c.stream, a,
                                1.0f / (float)c.N);
         else

@@ -1,0 +1,45 @@
+"""Mixed-form solves at radial resolutions without a compiled column length:
+columns padded with identity rows to a multiple of 16, at the smallest and
+largest N, at whole multiples of 16 and one row to either side, with partial
+blocks of harmonics, against the plain form's LDS-column solves.
+
+Both forms solve in FP64 and differ in the FP32 nonlinear terms N, of which
+dt N enters the state.  dt |N| < |x| here, so the states differ by less than
+one FP32 rounding, 2^-24 = 6e-8, a step; a wrong row of a solve shows at the
+order of its value."""
+import numpy as np
+import pytest
+
+from lsd import make_config, seeded_state, MIXED_F32, PLAIN_F64
+from lsd.gpu import Context
+
+pytestmark = pytest.mark.gpu
+
+
+def run(cfg, state):
+    g = Context(cfg)
+    g.set_state(state)
+    ev = g.step(2).evaluations
+    out = [g.get_coll(k) for k in range(6)]
+    v = g.variants()["solve"]
+    g.close()
+    return out, ev, v
+
+
+SIZES = [7, 15, 16, 17, 31, 40, 49, 63, 79, 80, 81, 95, 97, 111, 112, 113, 127, 128]
+
+
+@pytest.mark.parametrize("N", SIZES)
+@pytest.mark.parametrize("kw", [{}, {"rot": 1, "Nic": 8, "vel_bc": 2}], ids=["shell", "inner core"])
+def test_padded_columns(N, kw):
+    N = max(N, kw.get("Nic", 0))  # an inner core has at most N rows
+    def cfg(p):
+        return make_config(L=40, M=36, N=N, comp=1, Ra_comp=2.0e4, dt=1e-7, precision=p, **kw)
+    st = seeded_state(cfg(PLAIN_F64), 7, 1e-3)
+    a, ea, va = run(cfg(MIXED_F32), st)
+    b, eb, _ = run(cfg(PLAIN_F64), st)
+    assert va == 2 and ea == eb
+    for k in range(6):
+        den = np.sqrt((b[k][0] ** 2).sum() + (b[k][1] ** 2).sum())
+        num = np.sqrt(((a[k][0] - b[k][0]) ** 2).sum() + ((a[k][1] - b[k][1]) ** 2).sum())
+        assert num <= 2 * 2.0 ** -24 * den, (k, num / den)
