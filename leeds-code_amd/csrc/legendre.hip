@@ -20,12 +20,12 @@
 // Analysis (modules/transform.fftw3.F90:527-602, 825-949).  The forward FFT
 // leaves folded data G_p[j, c] (north+south, south-north), contracted as
 // D[k, c] = sum_j Tw[j, k] G[j, c] with the quadrature-weighted tables.  In
-// k_ana a workgroup takes one slot and 32 columns, stages 16-theta chunks of
+// k_ana (FP32, odd Th2 and the LDS-staged variant) a workgroup takes one slot and 32 columns, stages 16-theta chunks of
 // G through LDS, and each wave contracts 16-harmonic tiles of one parity
 // class against them, with the tables stored [j][h] and each slot's even-k
 // harmonics before its odd-k ones, so table reads and result writes are
-// 128-byte runs.  The FP32 form k_ana4 (below, for even Th2) reads both
-// operands 16 bytes per lane without LDS.
+// 128-byte runs.  The FP64 form k_ana8 and the FP32 form k_ana4 (below, for
+// even Th2) read their operands straight into registers, without LDS.
 #include <type_traits>
 
 #include "lsd_internal.h"
@@ -921,7 +921,7 @@ template <typename T>
 struct AnaArgs {
     int N, Th2, M, H;
     int ncc, ngroups;  // column chunks per job, slots
-    int njob;
+    int njob, maxhb;       // jobs, harmonic blocks of the longest class (k_ana8)
     const Slot* slots;
     const int* order;
     const T* tP;   // gwP        [Th2][H] (parity-grouped h)
@@ -941,10 +941,10 @@ constexpr int ANA_TPW = 4;     // max harmonic tiles per wave
 
 // VEC: q, s, t from three folded fields (tra_rtp2qst); else one field
 // (tra_phys2spec).  Workgroup: 4 waves, one slot, 32 columns.
-// FP32: two waves per SIMD (the compiler then fits the vector kind in 168
-// registers, without spills); FP64 keeps the whole register file
+// Two waves per SIMD: the compiler then fits the vector kind in 168
+// registers, without spills.
 template <typename T, bool VEC>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
 k_ana(AnaArgs<T> a) {
     typedef typename Mfma<T>::acc acc_t;
     constexpr int NF = VEC ? 3 : 1;
@@ -1089,7 +1089,7 @@ k_ana(AnaArgs<T> a) {
         }
     }
     // the lane holds class-local rows 16*kt + mrow of columns c0 + 16cb + l16
-    // (mrow = q4 + 4r for the FP64 instruction, 4q4 + r for FP32)
+    // (mrow = 4q4 + r)
 #pragma unroll
     for (int t = 0; t < ANA_TPW; t++) {
         const int tile = wave + 4 * t;
@@ -1099,7 +1099,7 @@ k_ana(AnaArgs<T> a) {
         const int ncls = par ? n_odd : n_even;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            const int kc = kt * 16 + (sizeof(T) == 8 ? q4 + 4 * r : 4 * q4 + r);
+            const int kc = kt * 16 + acc_row<T>(q4, r);
             if (kc >= ncls) continue;
             const size_t h = (size_t)s.h0 + 2 * kc + par;
 #pragma unroll
@@ -1118,6 +1118,158 @@ k_ana(AnaArgs<T> a) {
             }
         }
     }
+}
+
+// ------------------------------------------------------------ FP64 analysis
+//
+// The same contractions without LDS or barriers.  A wave takes one (slot,
+// parity class, up to A8_TP tiles of 16 harmonics) and 16 shells, and
+// contracts over all theta, four per K step as k_ana does and in its order of
+// products, so the sums are the same bit for bit:
+// * the A operands are the tables, 8 bytes per lane and tile (128-byte runs);
+// * the B operands are the folded data, one 16-byte load per lane for (re, im)
+//   of the lane's shell at one theta: both column tiles of the MFMA, so the i
+//   rotations are a swap within the lane;
+// * the operands of the next K step but one are loaded while a step's
+//   products run.
+// The two waves of a workgroup take the two classes of the same shells, which
+// read the same folded rows.
+// Bound: three tiles and 30 MFMAs (1920 cycles) a step against 9.5 KB of
+// operands, from L2 mostly; the barriers and single wave per SIMD of the
+// LDS-staged form left the matrix cores idle 4 cycles in 5.  L = M = 170,
+// N = 96, both vector fields: 483 -> 264 us (27 of 73 TFLOP/s), scalars 75 ->
+// 70 us; L = M = 32, N = 32: 11 -> 6.6 us.
+constexpr int A8_TP = 3;   // harmonic tiles per wave at most
+constexpr int A8_SH = 16;  // shells per wave
+constexpr int A8_NB = 2;   // operand buffers
+
+template <bool VEC, int TP>
+struct A8Ops {
+    static constexpr int NG = VEC ? 5 : 1, NT = VEC ? 3 : 1;
+    double2 g[NG];       // r(p), theta(1-p), phi(p), theta(p), phi(1-p)
+    double w[TP][NT];    // tables P, L, S
+};
+
+// tile0, tile0 + 1, ... of class par of slot s, shells 16 sb to 16 sb + 15
+template <bool VEC, int TP>
+__device__ __forceinline__ void ana8_item(const AnaArgs<double>& a, const Slot& s, int job, int sb, int par,
+                                          int tile0) {
+    typedef A8Ops<VEC, TP> Ops;
+    constexpr int NO = VEC ? 3 : 1;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, q4 = lane >> 4;
+    const int n_even = (s.len + 1) / 2, ncls = par ? s.len / 2 : n_even;
+    const size_t col0 = (size_t)s.h0 + (par ? n_even : 0);
+    int kcol[TP];
+#pragma unroll
+    for (int t = 0; t < TP; t++) kcol[t] = min((tile0 + t) * 16 + l16, ncls - 1);
+    const int n = sb * A8_SH + l16, nc = min(n, a.N - 1);
+    const size_t row = ((size_t)nc * a.M + s.mfft) * 2 * a.Th2;
+    const size_t rp = row + (size_t)par * a.Th2, ro = row + (size_t)(1 - par) * a.Th2;
+    const double2* g1 = reinterpret_cast<const double2*>(pickj(a.g1, job));
+    const double2* g2 = VEC ? reinterpret_cast<const double2*>(pickj(a.g2, job)) : nullptr;
+    const double2* g3 = VEC ? reinterpret_cast<const double2*>(pickj(a.g3, job)) : nullptr;
+    auto load = [&](Ops& op, int j0) {
+        const int j = j0 + q4, jc = min(j, a.Th2 - 1);
+        op.g[0] = g1[rp + jc];
+        if constexpr (VEC) {
+            op.g[1] = g2[ro + jc];
+            op.g[2] = g3[rp + jc];
+            op.g[3] = g2[rp + jc];
+            op.g[4] = g3[ro + jc];
+        }
+        const size_t trow = (size_t)jc * a.H + col0;
+#pragma unroll
+        for (int t = 0; t < TP; t++) {
+            op.w[t][0] = a.tP[trow + kcol[t]];
+            if constexpr (VEC) {
+                op.w[t][1] = a.tL[trow + kcol[t]];
+                op.w[t][2] = a.tS[trow + kcol[t]];
+            }
+        }
+    };
+    v4d acc[TP][NO][2];
+#pragma unroll
+    for (int t = 0; t < TP; t++)
+#pragma unroll
+        for (int o = 0; o < NO; o++) acc[t][o][0] = acc[t][o][1] = v4d{0, 0, 0, 0};
+    auto step = [&](Ops& op, int j0) {
+        if (j0 + 4 > a.Th2) {  // the last step's theta past Th2 add nothing
+            const bool jv = j0 + q4 < a.Th2;
+#pragma unroll
+            for (int f = 0; f < Ops::NG; f++) {
+                op.g[f].x = jv ? op.g[f].x : 0.0;
+                op.g[f].y = jv ? op.g[f].y : 0.0;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TP; t++) {
+            const double wP = op.w[t][0];
+            acc[t][0][0] = Mfma<double>::run(wP, op.g[0].x, acc[t][0][0]);
+            acc[t][0][1] = Mfma<double>::run(wP, op.g[0].y, acc[t][0][1]);
+            if constexpr (VEC) {
+                const double wL = op.w[t][Ops::NT - 2], wS = op.w[t][Ops::NT - 1];
+                const double2 y2o = op.g[Ops::NG - 4], y3s = op.g[Ops::NG - 3], y2s = op.g[Ops::NG - 2],
+                              y3o = op.g[Ops::NG - 1];
+                // s += Y2o gl - i Y3s gs, t += i Y2s gs + Y3o gl
+                acc[t][NO - 2][0] = Mfma<double>::run(wL, y2o.x, acc[t][NO - 2][0]);
+                acc[t][NO - 2][1] = Mfma<double>::run(wL, y2o.y, acc[t][NO - 2][1]);
+                acc[t][NO - 1][0] = Mfma<double>::run(wS, -y2s.y, acc[t][NO - 1][0]);
+                acc[t][NO - 1][1] = Mfma<double>::run(wS, y2s.x, acc[t][NO - 1][1]);
+                acc[t][NO - 2][0] = Mfma<double>::run(wS, y3s.y, acc[t][NO - 2][0]);
+                acc[t][NO - 2][1] = Mfma<double>::run(wS, -y3s.x, acc[t][NO - 2][1]);
+                acc[t][NO - 1][0] = Mfma<double>::run(wL, y3o.x, acc[t][NO - 1][0]);
+                acc[t][NO - 1][1] = Mfma<double>::run(wL, y3o.y, acc[t][NO - 1][1]);
+            }
+        }
+    };
+    Ops ops[A8_NB];
+#pragma unroll
+    for (int u = 0; u < A8_NB; u++) load(ops[u], 4 * u);
+    for (int j0 = 0; j0 < a.Th2; j0 += 4 * A8_NB) {
+#pragma unroll
+        for (int u = 0; u < A8_NB; u++) {
+            if (j0 + 4 * u < a.Th2) step(ops[u], j0 + 4 * u);
+            load(ops[u], j0 + 4 * (u + A8_NB));
+        }
+    }
+    if (n >= a.N) return;
+    const bool m0 = s.m == 0;
+#pragma unroll
+    for (int t = 0; t < TP; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int kc = (tile0 + t) * 16 + acc_row<double>(q4, r);
+            if (kc >= ncls) continue;
+            const size_t o = ((size_t)s.h0 + 2 * kc + par) * a.N + n;
+            // Im of m = 0 is zero, but the reference leaves q%Im(m=0) as summed
+#pragma unroll
+            for (int f = 0; f < NO; f++) {
+                double* out = f == 0 ? pickj(a.o1, job) : f == 1 ? pickj(a.o2, job) : pickj(a.o3, job);
+                const bool zero_im = m0 && (!VEC || f > 0);
+                reinterpret_cast<double2*>(out)[o] =
+                    make_double2(acc[t][f][0][r], zero_im ? 0.0 : acc[t][f][1][r]);
+            }
+        }
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) k_ana8(AnaArgs<double> a) {
+    // groups: slots, longest first; members (job, harmonic block, shell block)
+    // on one XCD, reading the same tables
+    const BlockId bid = decode_block(a.ngroups, a.njob * a.maxhb * a.ncc);
+    if (!bid.valid) return;
+    const Slot s = a.slots[uniform(a.order[bid.group])];
+    const int job = bid.cc / (a.maxhb * a.ncc), rest = bid.cc - job * a.maxhb * a.ncc;
+    const int hb = rest / a.ncc, sb = rest - hb * a.ncc;
+    const int par = uniform(threadIdx.x >> 6);
+    // the class's tiles in equal shares of at most A8_TP
+    const int ncls = par ? s.len / 2 : (s.len + 1) / 2;
+    const int tiles = (ncls + 15) / 16, nb = (tiles + A8_TP - 1) / A8_TP;
+    if (hb >= nb) return;
+    const int t0 = tiles * hb / nb, nt = tiles * (hb + 1) / nb - t0;
+    if (nt == 3) ana8_item<VEC, 3>(a, s, job, sb, par, t0);
+    else if (nt == 2) ana8_item<VEC, 2>(a, s, job, sb, par, t0);
+    else ana8_item<VEC, 1>(a, s, job, sb, par, t0);
 }
 
 // ----------------------------------------------------- FP32 analysis (mixed forms)
@@ -1401,9 +1553,17 @@ static int ana_launch(Ctx& c, int kind, int njob, const T* tP, const T* tL, cons
     a.ncc = (2 * c.N + ANA_COLS - 1) / ANA_COLS;
     a.ngroups = c.nslot;
     a.njob = njob;
-    dim3 grid(grid_blocks(a.ngroups, a.ncc * njob));
-    if (kind == ANA_SCALAR) hipLaunchKernelGGL((k_ana<T, false>), grid, dim3(256), 0, c.stream, a);
-    else hipLaunchKernelGGL((k_ana<T, true>), grid, dim3(256), 0, c.stream, a);
+    a.maxhb = (((maxlen + 1) / 2 + 15) / 16 + A8_TP - 1) / A8_TP;
+    if constexpr (std::is_same<T, double>::value) {
+        static_assert(2 * A8_SH == ANA_COLS, "one shell block per column chunk");
+        const dim3 grid(grid_blocks(a.ngroups, a.ncc * a.maxhb * njob));
+        if (kind == ANA_SCALAR) hipLaunchKernelGGL(k_ana8<false>, grid, dim3(128), 0, c.stream, a);
+        else hipLaunchKernelGGL(k_ana8<true>, grid, dim3(128), 0, c.stream, a);
+    } else {
+        const dim3 grid(grid_blocks(a.ngroups, a.ncc * njob));
+        if (kind == ANA_SCALAR) hipLaunchKernelGGL((k_ana<T, false>), grid, dim3(256), 0, c.stream, a);
+        else hipLaunchKernelGGL((k_ana<T, true>), grid, dim3(256), 0, c.stream, a);
+    }
     LSD_HIP(hipGetLastError());
     return LSD_OK;
 }

@@ -1,0 +1,21 @@
+"""FP64 Legendre sums at the edges of their tiles: harmonic counts of a parity
+class around the 16 of a tile and the 48 of a wave, shells around 16, theta
+counts around the 4 of a step, the 16 and the 32 of a tile, M = 1 and every
+fourth m.  The nonlinear terms of one timestep against the C oracle, relative
+to each field's norm within 1e-11 (the bound of the other parity tests: about
+L roundings of 1.1e-16 a sum, through two sums and two transforms)."""
+import pytest
+
+from lsd import make_config, PLAIN_F64
+from test_gpu_physwave import compare
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("L,M,Mp,N,Th,Ph", [
+    (8, 1, 1, 15, 14, 8), (32, 32, 1, 16, 48, 96), (33, 32, 1, 17, 50, 96), (64, 64, 1, 31, 96, 192),
+    (95, 30, 1, 33, 144, 96), (97, 12, 4, 9, 146, 48), (98, 32, 1, 32, 150, 96), (130, 16, 1, 24, 196, 48),
+    (194, 8, 1, 16, 292, 36), (256, 6, 2, 8, 386, 24)])
+def test_tiles(L, M, Mp, N, Th, Ph):
+    compare(make_config(L=L, M=M, Mp=Mp, N=N, Th=Th, Ph=Ph, comp=1, dt=1e-4, precision=PLAIN_F64, Ra_comp=2.0e4,
+                        dterr=1e30), 1e-11)
