@@ -1,0 +1,151 @@
+// Copies between a caller's arrays and the device through pinned chunks.
+//
+// The caller's arrays are pageable.  A plain copy of one pins its pages or
+// moves them through the runtime's own staging with one thread, and a result
+// array's pages are mapped by that thread as it first writes them, which
+// bounds the copy at about 6-8 GB/s against the 55 GB/s of the link.  Here
+// HC_THREADS threads (the caller's among them) each own two pinned chunks:
+// while one chunk is on the link the other is copied to or from the caller's
+// array, so the page mapping and the host copies of the threads run side by
+// side with the transfers.  The chunks belong to one context or network and
+// are freed with it.  Three components to the grid and back at L = M = 64,
+// N = 64, 96 x 192 (69 MB): 5.6 -> 3.4 ms; the closure network on 57792 rows
+// of 92 values: 0.98-1.05 -> 0.96 ms, its first call 1.8 -> 1.2 ms.
+#include <cstring>
+#include <system_error>
+#include <thread>
+
+#include "lsd_internal.h"
+
+namespace lsd {
+
+constexpr int HC_THREADS = 4;  // eight gain nothing: mapping the pages takes turns
+constexpr size_t HC_CHUNK = size_t(1) << 20;
+// below this the threads' start (about 50 us) costs more than they save
+constexpr size_t HC_MIN = size_t(2) << 20;
+
+int HostStage::reserve() {
+    if (buf) return LSD_OK;
+    for (hipEvent_t& e : ev)
+        if (!e) LSD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    LSD_HIP(hipHostMalloc((void**)&buf, 2 * HC_THREADS * HC_CHUNK, hipHostMallocDefault));
+    return LSD_OK;
+}
+
+void HostStage::release() {
+    static_assert(sizeof(ev) / sizeof(ev[0]) == 2 * HC_THREADS, "two chunks a thread");
+    if (buf) (void)hipHostFree(buf);
+    buf = nullptr;
+    for (hipEvent_t& e : ev) {
+        if (e) (void)hipEventDestroy(e);
+        e = nullptr;
+    }
+}
+
+// Chunk q of the parts: host and device address and length.
+struct HcChunk {
+    char* host;
+    char* dev;
+    size_t n;
+};
+static HcChunk chunk_at(const HostPart* parts, int np, size_t q) {
+    for (int k = 0; k < np; k++) {
+        const size_t nq = (parts[k].bytes + HC_CHUNK - 1) / HC_CHUNK;
+        if (q < nq) {
+            const size_t at = q * HC_CHUNK;
+            return {(char*)parts[k].host + at, (char*)parts[k].dev + at, std::min(HC_CHUNK, parts[k].bytes - at)};
+        }
+        q -= nq;
+    }
+    return {nullptr, nullptr, 0};
+}
+
+// The chunks t, t + HC_THREADS, ... of one thread.
+static hipError_t copy_share(HostStage& st, int device, hipStream_t stream, const HostPart* parts, int np, size_t nq,
+                             int t, bool to_host) {
+    hipError_t e = hipSetDevice(device);
+    if (e != hipSuccess) return e;
+    HcChunk prev{nullptr, nullptr, 0};
+    int slot = 2 * t;
+    for (size_t q = t; q < nq; q += HC_THREADS, slot ^= 1) {
+        const HcChunk c = chunk_at(parts, np, q);
+        char* b = st.buf + slot * HC_CHUNK;
+        if (to_host) {
+            if ((e = hipMemcpyAsync(b, c.dev, c.n, hipMemcpyDeviceToHost, stream)) != hipSuccess) return e;
+            if ((e = hipEventRecord(st.ev[slot], stream)) != hipSuccess) return e;
+            if (prev.n) {
+                if ((e = hipEventSynchronize(st.ev[slot ^ 1])) != hipSuccess) return e;
+                memcpy(prev.host, st.buf + (slot ^ 1) * HC_CHUNK, prev.n);
+            }
+            prev = c;
+        } else {
+            // the chunk's last copy has left it (a new event counts as done)
+            if ((e = hipEventSynchronize(st.ev[slot])) != hipSuccess) return e;
+            memcpy(b, c.host, c.n);
+            if ((e = hipMemcpyAsync(c.dev, b, c.n, hipMemcpyHostToDevice, stream)) != hipSuccess) return e;
+            if ((e = hipEventRecord(st.ev[slot], stream)) != hipSuccess) return e;
+        }
+    }
+    if (prev.n) {
+        if ((e = hipEventSynchronize(st.ev[slot ^ 1])) != hipSuccess) return e;
+        memcpy(prev.host, st.buf + (slot ^ 1) * HC_CHUNK, prev.n);
+    }
+    return hipSuccess;
+}
+
+// Memory the runtime does not know.  Pinned, managed or device memory in a
+// caller's array goes straight to the link.
+static bool pageable(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
+// to_host: on return the host arrays hold the data; otherwise the host arrays
+// have been read and the copies are in the stream's order.
+int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host) {
+    size_t total = 0, nq = 0;
+    bool chunks = true;
+    for (int k = 0; k < np; k++) {
+        if (!parts[k].host) {
+            set_error("null host array");
+            return LSD_E_HIP;
+        }
+        total += parts[k].bytes;
+        nq += (parts[k].bytes + HC_CHUNK - 1) / HC_CHUNK;
+    }
+    for (int k = 0; k < np && total >= HC_MIN; k++) chunks = chunks && pageable(parts[k].host);
+    if (total < HC_MIN || !chunks) {
+        for (int k = 0; k < np; k++)
+            LSD_HIP(hipMemcpyAsync(to_host ? parts[k].host : parts[k].dev, to_host ? parts[k].dev : parts[k].host,
+                                   parts[k].bytes, to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, stream));
+        if (to_host) LSD_HIP(hipStreamSynchronize(stream));
+        return LSD_OK;
+    }
+    const int rc = st.reserve();
+    if (rc) return rc;
+    int device = 0;
+    LSD_HIP(hipGetDevice(&device));
+    hipError_t err[HC_THREADS];
+    std::thread th[HC_THREADS];
+    auto share = [&](int t) { err[t] = copy_share(st, device, stream, parts, np, nq, t, to_host); };
+    for (int t = 1; t < HC_THREADS; t++) {
+        try {
+            th[t] = std::thread(share, t);
+        } catch (const std::system_error&) {
+            // no thread to be had: the caller's takes the share below
+        }
+    }
+    share(0);
+    for (int t = 1; t < HC_THREADS; t++) {
+        if (th[t].joinable()) th[t].join();
+        else share(t);
+    }
+    for (int t = 0; t < HC_THREADS; t++) LSD_HIP(err[t]);
+    return LSD_OK;
+}
+
+}  // namespace lsd

@@ -1138,7 +1138,7 @@ k_ana(AnaArgs<T> a) {
 // operands, from L2 mostly; the barriers and single wave per SIMD of the
 // LDS-staged form left the matrix cores idle 4 cycles in 5.  L = M = 170,
 // N = 96, both vector fields: 483 -> 264 us (27 of 73 TFLOP/s), scalars 75 ->
-// 70 us; L = M = 32, N = 32: 11 -> 6.6 us.
+// 70 us; L = M = 32, N = 32: 14.6 -> 6.6 us.
 constexpr int A8_TP = 3;   // harmonic tiles per wave at most
 constexpr int A8_SH = 16;  // shells per wave
 constexpr int A8_NB = 2;   // operand buffers

@@ -121,6 +121,7 @@ static void release(Ctx* c) {
     if (c->h_partial) (void)hipHostFree(c->h_partial);
     if (c->h_icpartial) (void)hipHostFree(c->h_icpartial);
     if (c->h_cfl) (void)hipHostFree(c->h_cfl);
+    c->stage.release();
     for (hipEvent_t e : c->prof_events) (void)hipEventDestroy(e);
     drop_graphs(*c);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -555,15 +556,63 @@ static double2* folded(Ctx& c, int k) { return c.d_folded + (size_t)k * c.folded
 static double* phys(Ctx& c, int k) { return c.d_phys + (size_t)k * c.phys_elems(); }
 static double* nlphys(Ctx& c, int k) { return c.d_nlphys + (size_t)k * c.phys_elems(); }
 
+// Re and Im of one coll-sized array, to or from the two halves of tmp.
+static int copy_pair(Ctx& c, const double* re, const double* im, double* tmp, bool to_host) {
+    const size_t b = sizeof(double) * c.coll_elems();
+    const HostPart parts[2] = {{const_cast<double*>(re), tmp, b}, {const_cast<double*>(im), tmp + c.coll_elems(), b}};
+    return host_copy(c.stage, c.stream, parts, 2, to_host);
+}
+
 // Two real coll arrays on the device for a field on its way to or from the
 // host: the synthesis inputs, which every evaluation writes before it reads
 // them.  Splitting Re and Im here instead of on the host (a zero-filled copy,
-// then a loop over it) takes reading the six fields from 42 to 25 ms at
-// L = M = 170, N = 96 and from 160 to 63-80 ms at L = M = 256, N = 128; what is
-// left is the copy to pageable memory.
+// then a loop over it) took reading the six fields from 42 to 25 ms at
+// L = M = 170, N = 96 and from 160 to 63-80 ms at L = M = 256, N = 128; the
+// pinned chunks of host_copy then take it to 20 and 60 ms.
 static double* coll_staging(Ctx& c) {
     static_assert(SI_COUNT >= 1, "at least one double2 coll array");
     return reinterpret_cast<double*>(c.d_spec_in);
+}
+
+// nf spectral arrays (Re and Im each) in one copy.  They are staged in the
+// analysis outputs on their way in and in the synthesis inputs on their way
+// out (2*H*N doubles each), neither of which is in use then.
+constexpr int TRA_MAX = 3;
+static double* spec_staging(Ctx& c, int k, bool to_host) {
+    static_assert(TRA_MAX <= SO_COUNT && TRA_MAX <= SI_COUNT, "a buffer for each array");
+    return reinterpret_cast<double*>(to_host ? spec_in(c, k) : spec_out(c, k));
+}
+static int copy_spec(Ctx& c, int nf, const double* const* re, const double* const* im, bool to_host) {
+    const size_t HN = c.coll_elems();
+    HostPart parts[2 * TRA_MAX];
+    for (int k = 0; k < nf; k++) {
+        double* tmp = spec_staging(c, k, to_host);
+        parts[2 * k] = {const_cast<double*>(re[k]), tmp, sizeof(double) * HN};
+        parts[2 * k + 1] = {const_cast<double*>(im[k]), tmp + HN, sizeof(double) * HN};
+    }
+    return host_copy(c.stage, c.stream, parts, 2 * nf, to_host);
+}
+static int upload_spec(Ctx& c, int nf, const double* const* re, const double* const* im, double2* const* dst) {
+    int rc = copy_spec(c, nf, re, im, false);
+    for (int k = 0; k < nf && !rc; k++) {
+        double* tmp = spec_staging(c, k, false);
+        rc = launch_layout_spec2coll(c, tmp, tmp + c.coll_elems(), dst[k]);
+    }
+    return rc;
+}
+static int download_spec(Ctx& c, int nf, const double2* const* src, double* const* re, double* const* im) {
+    for (int k = 0; k < nf; k++) {
+        double* tmp = spec_staging(c, k, true);
+        int rc = launch_layout_coll2spec(c, src[k], tmp, tmp + c.coll_elems());
+        if (rc) return rc;
+    }
+    return copy_spec(c, nf, re, im, true);
+}
+// nf grid arrays to or from phys buffers 0, 1, ...
+static int copy_phys(Ctx& c, int nf, const double* const* p, bool to_host) {
+    HostPart parts[TRA_MAX];
+    for (int k = 0; k < nf; k++) parts[k] = {const_cast<double*>(p[k]), phys(c, k), sizeof(double) * c.phys_elems()};
+    return host_copy(c.stage, c.stream, parts, nf, to_host);
 }
 
 #define RC(x)             \
@@ -1258,10 +1307,8 @@ int lsd_set_coll(lsd_ctx* ctx, int field, const double* re, const double* im) {
     }
     const size_t HN = c.coll_elems();
     double* tmp = lsd::coll_staging(c);
-    LSD_HIP(hipMemcpyAsync(tmp, re, sizeof(double) * HN, hipMemcpyHostToDevice, c.stream));
-    LSD_HIP(hipMemcpyAsync(tmp + HN, im, sizeof(double) * HN, hipMemcpyHostToDevice, c.stream));
-    int rc = lsd::launch_merge_coll(c, tmp, tmp + HN, c.d_f[field]);
-    if (rc) return rc;
+    int rc = lsd::copy_pair(c, re, im, tmp, false);
+    if (rc || (rc = lsd::launch_merge_coll(c, tmp, tmp + HN, c.d_f[field]))) return rc;
     LSD_HIP(hipStreamSynchronize(c.stream));
     return LSD_OK;
 }
@@ -1465,11 +1512,7 @@ int lsd_get_coll(lsd_ctx* ctx, int field, double* re, double* im) {
     const size_t HN = c.coll_elems();
     double* tmp = lsd::coll_staging(c);
     int rc = lsd::launch_split_coll(c, c.d_f[field], tmp, tmp + HN);
-    if (rc) return rc;
-    LSD_HIP(hipMemcpyAsync(re, tmp, sizeof(double) * HN, hipMemcpyDeviceToHost, c.stream));
-    LSD_HIP(hipMemcpyAsync(im, tmp + HN, sizeof(double) * HN, hipMemcpyDeviceToHost, c.stream));
-    LSD_HIP(hipStreamSynchronize(c.stream));
-    return LSD_OK;
+    return rc ? rc : lsd::copy_pair(c, re, im, tmp, true);
 }
 
 int lsd_get_phys(lsd_ctx* ctx, int field, double* p) {
@@ -1478,10 +1521,8 @@ int lsd_get_phys(lsd_ctx* ctx, int field, double* p) {
         lsd::set_error("lsd_get_phys: bad field or null pointer");
         return LSD_E_ARG;
     }
-    LSD_HIP(hipMemcpyAsync(p, lsd::phys(c, field), sizeof(double) * c.phys_elems(), hipMemcpyDeviceToHost,
-                           c.stream));
-    LSD_HIP(hipStreamSynchronize(c.stream));
-    return LSD_OK;
+    const lsd::HostPart part = {p, lsd::phys(c, field), sizeof(double) * c.phys_elems()};
+    return lsd::host_copy(c.stage, c.stream, &part, 1, true);
 }
 
 int lsd_get_table(lsd_ctx* ctx, int table, double* out) {
@@ -1724,30 +1765,6 @@ int lsd_set_dt(lsd_ctx* ctx, double dt) {
 
 // ---------------------------------------------------- drop-in transforms
 
-static int upload_spec(Ctx& c, const double* re, const double* im, double2* dst) {
-    size_t HN = c.coll_elems();
-    double* tmp = reinterpret_cast<double*>(lsd::nlphys(c, 0));  // staging, >= 2*H*N doubles
-    LSD_HIP(hipMemcpyAsync(tmp, re, sizeof(double) * HN, hipMemcpyHostToDevice, c.stream));
-    LSD_HIP(hipMemcpyAsync(tmp + HN, im, sizeof(double) * HN, hipMemcpyHostToDevice, c.stream));
-    return lsd::launch_layout_spec2coll(c, tmp, tmp + HN, dst);
-}
-
-static int download_spec(Ctx& c, const double2* src, double* re, double* im) {
-    size_t HN = c.coll_elems();
-    double* tmp = reinterpret_cast<double*>(lsd::nlphys(c, 0));
-    int rc = lsd::launch_layout_coll2spec(c, src, tmp, tmp + HN);
-    if (rc) return rc;
-    LSD_HIP(hipMemcpyAsync(re, tmp, sizeof(double) * HN, hipMemcpyDeviceToHost, c.stream));
-    LSD_HIP(hipMemcpyAsync(im, tmp + HN, sizeof(double) * HN, hipMemcpyDeviceToHost, c.stream));
-    LSD_HIP(hipStreamSynchronize(c.stream));
-    return LSD_OK;
-}
-
-static int download_phys(Ctx& c, int k, double* p) {
-    LSD_HIP(hipMemcpyAsync(p, lsd::phys(c, k), sizeof(double) * c.phys_elems(), hipMemcpyDeviceToHost, c.stream));
-    return LSD_OK;
-}
-
 // Synthesis -> analysis round trip at the Fourier level in the context's
 // precision (FP64, FP32 or BF16x3 Legendre kernels).
 int lsd_sht_roundtrip(lsd_ctx* ctx, int kind, const double* in, double* out) {
@@ -1810,26 +1827,22 @@ int lsd_tra_spec2phys(lsd_ctx* ctx, const double* s_re, const double* s_im, doub
     CTX_OR_FAIL(ctx);
     int rc;
     double2* in = lsd::spec_in(c, lsd::SI_DC);
-    if ((rc = upload_spec(c, s_re, s_im, in))) return rc;
+    if ((rc = lsd::upload_spec(c, 1, &s_re, &s_im, &in))) return rc;
     if ((rc = lsd::launch_synthesis(c, lsd::SYN_SCALAR, in, nullptr, lsd::fourier(c, 0), nullptr))) return rc;
     if ((rc = lsd::launch_fft_c2r(c, lsd::fourier(c, 0), lsd::phys(c, 0), 1))) return rc;
-    if ((rc = download_phys(c, 0, p))) return rc;
-    LSD_HIP(hipStreamSynchronize(c.stream));
-    return LSD_OK;
+    return lsd::copy_phys(c, 1, &p, true);
 }
 
 int lsd_tra_grad(lsd_ctx* ctx, const double* s_re, const double* s_im, double* t, double* p) {
     CTX_OR_FAIL(ctx);
     int rc;
     double2* in = lsd::spec_in(c, lsd::SI_DC);
-    if ((rc = upload_spec(c, s_re, s_im, in))) return rc;
+    if ((rc = lsd::upload_spec(c, 1, &s_re, &s_im, &in))) return rc;
     if ((rc = lsd::launch_synthesis(c, lsd::SYN_GRAD, in, nullptr, lsd::fourier(c, 0), lsd::fourier(c, 1))))
         return rc;
     if ((rc = lsd::launch_fft_c2r(c, lsd::fourier(c, 0), lsd::phys(c, 0), 2))) return rc;
-    if ((rc = download_phys(c, 0, t))) return rc;
-    if ((rc = download_phys(c, 1, p))) return rc;
-    LSD_HIP(hipStreamSynchronize(c.stream));
-    return LSD_OK;
+    const double* out[2] = {t, p};
+    return lsd::copy_phys(c, 2, out, true);
 }
 
 int lsd_tra_qst2rtp(lsd_ctx* ctx, const double* q_re, const double* q_im, const double* s_re, const double* s_im,
@@ -1839,37 +1852,35 @@ int lsd_tra_qst2rtp(lsd_ctx* ctx, const double* q_re, const double* q_im, const 
     double2* q = lsd::spec_in(c, lsd::SI_UQ);
     double2* s = lsd::spec_in(c, lsd::SI_US);
     double2* t = lsd::spec_in(c, lsd::SI_UT);
-    if ((rc = upload_spec(c, q_re, q_im, q)) || (rc = upload_spec(c, s_re, s_im, s)) ||
-        (rc = upload_spec(c, t_re, t_im, t)))
-        return rc;
+    const double* re[3] = {q_re, s_re, t_re};
+    const double* im[3] = {q_im, s_im, t_im};
+    double2* in[3] = {q, s, t};
+    if ((rc = lsd::upload_spec(c, 3, re, im, in))) return rc;
     if ((rc = lsd::launch_synthesis(c, lsd::SYN_SCALAR, q, nullptr, lsd::fourier(c, 0), nullptr))) return rc;
     if ((rc = lsd::launch_synthesis(c, lsd::SYN_VECTOR, s, t, lsd::fourier(c, 1), lsd::fourier(c, 2)))) return rc;
     if ((rc = lsd::launch_fft_c2r(c, lsd::fourier(c, 0), lsd::phys(c, 0), 3))) return rc;
-    if ((rc = download_phys(c, 0, r)) || (rc = download_phys(c, 1, th)) || (rc = download_phys(c, 2, ph))) return rc;
-    LSD_HIP(hipStreamSynchronize(c.stream));
-    return LSD_OK;
+    const double* out[3] = {r, th, ph};
+    return lsd::copy_phys(c, 3, out, true);
 }
 
 int lsd_tra_phys2spec(lsd_ctx* ctx, const double* p, double* s_re, double* s_im) {
     CTX_OR_FAIL(ctx);
     int rc;
     double* x = lsd::phys(c, 0);
-    LSD_HIP(hipMemcpyAsync(x, p, sizeof(double) * c.phys_elems(), hipMemcpyHostToDevice, c.stream));
+    if ((rc = lsd::copy_phys(c, 1, &p, false))) return rc;
     if ((rc = lsd::launch_fft_r2c_fold(c, x, lsd::folded(c, 0), 1))) return rc;
     double2* o = lsd::spec_out(c, lsd::SO_C);
     if ((rc = lsd::launch_analysis(c, lsd::ANA_SCALAR, lsd::folded(c, 0), nullptr, nullptr, o, nullptr, nullptr)))
         return rc;
-    return download_spec(c, o, s_re, s_im);
+    return lsd::download_spec(c, 1, &o, &s_re, &s_im);
 }
 
 int lsd_tra_rtp2qst(lsd_ctx* ctx, const double* r, const double* th, const double* ph, double* q_re, double* q_im,
                     double* s_re, double* s_im, double* t_re, double* t_im) {
     CTX_OR_FAIL(ctx);
     int rc;
-    size_t np = c.phys_elems();
-    LSD_HIP(hipMemcpyAsync(lsd::phys(c, 0), r, sizeof(double) * np, hipMemcpyHostToDevice, c.stream));
-    LSD_HIP(hipMemcpyAsync(lsd::phys(c, 1), th, sizeof(double) * np, hipMemcpyHostToDevice, c.stream));
-    LSD_HIP(hipMemcpyAsync(lsd::phys(c, 2), ph, sizeof(double) * np, hipMemcpyHostToDevice, c.stream));
+    const double* in[3] = {r, th, ph};
+    if ((rc = lsd::copy_phys(c, 3, in, false))) return rc;
     if ((rc = lsd::launch_fft_r2c_fold(c, lsd::phys(c, 0), lsd::folded(c, 0), 3))) return rc;
     double2* o0 = lsd::spec_out(c, lsd::SO_UQ);
     double2* o1 = lsd::spec_out(c, lsd::SO_US);
@@ -1877,10 +1888,10 @@ int lsd_tra_rtp2qst(lsd_ctx* ctx, const double* r, const double* th, const doubl
     if ((rc = lsd::launch_analysis(c, lsd::ANA_VECTOR, lsd::folded(c, 0), lsd::folded(c, 1), lsd::folded(c, 2), o0,
                                    o1, o2)))
         return rc;
-    if ((rc = download_spec(c, o0, q_re, q_im)) || (rc = download_spec(c, o1, s_re, s_im)) ||
-        (rc = download_spec(c, o2, t_re, t_im)))
-        return rc;
-    return LSD_OK;
+    const double2* o[3] = {o0, o1, o2};
+    double* re[3] = {q_re, s_re, t_re};
+    double* im[3] = {q_im, s_im, t_im};
+    return lsd::download_spec(c, 3, o, re, im);
 }
 
 }  // extern "C"

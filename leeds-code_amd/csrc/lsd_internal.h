@@ -45,6 +45,21 @@ void harmonics(int L, int M, int Mp, std::vector<int>& hl, std::vector<int>& hm)
         }                                                                     \
     } while (0)
 
+// hostcopy.hip: pinned chunks for copies between a caller's pageable arrays
+// and the device, allocated at the first copy that uses them.
+struct HostStage {
+    char* buf = nullptr;
+    hipEvent_t ev[8] = {};
+    int reserve();
+    void release();
+};
+struct HostPart {
+    void* host;
+    void* dev;
+    size_t bytes;
+};
+int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host);
+
 // Stream-ordered scratch of a set-up or diagnostic call, returned to the
 // pool on every exit path (the call synchronises the stream before using
 // what the kernels wrote, so the free follows all uses).
@@ -196,6 +211,7 @@ struct Ctx {
     int solve_hb = 0;                  // harmonics per solve block
 
     // kernel variants (LSD_V_*), see lsd_set_variant
+    HostStage stage;                   // copies to and from the caller's arrays
     int var[LSD_V_COUNT] = {4, 8, 8, 0, 0};
     bool ana_wide_ok = false;          // the wide-load FP32 analysis applies (even Th2)
     bool solve_direct_ok = false;      // the two-pass solves apply (N in {32, 48, 64, 96})

@@ -556,6 +556,7 @@ struct lsd_mlp {
     int nin, width, nout;
     long np;
     hipStream_t stream = nullptr;
+    lsd::HostStage stage;  // copies to and from the caller's arrays
     float* p = nullptr;   // parameters
     float* g = nullptr;   // gradients
     float* m1 = nullptr;  // Adam moments
@@ -909,6 +910,7 @@ void lsd_mlp_destroy(lsd_mlp* m) {
     (void)hipFree(m->g);
     (void)hipFree(m->m1);
     (void)hipFree(m->m2);
+    m->stage.release();
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
 }
@@ -931,11 +933,11 @@ int lsd_mlp_forward(lsd_mlp* m, long rows, const float* x, float* y) {
     if (!m || !x || !y || rows < 1) { lsd::set_error("lsd_mlp_forward: bad arguments"); return LSD_E_ARG; }
     int rc = m->fused() ? mlp_io(m, rows) : mlp_rows(m, rows);
     if (rc) return rc;
-    LSD_HIP(hipMemcpyAsync(m->X, x, sizeof(float) * rows * m->nin, hipMemcpyHostToDevice, m->stream));
+    const lsd::HostPart in = {const_cast<float*>(x), m->X, sizeof(float) * rows * m->nin};
+    const lsd::HostPart out = {y, m->Y, sizeof(float) * rows * m->nout};
+    if ((rc = lsd::host_copy(m->stage, m->stream, &in, 1, false))) return rc;
     if ((rc = mlp_forward_dev(m, rows, m->X, false))) return rc;
-    LSD_HIP(hipMemcpyAsync(y, m->Y, sizeof(float) * rows * m->nout, hipMemcpyDeviceToHost, m->stream));
-    LSD_HIP(hipStreamSynchronize(m->stream));
-    return LSD_OK;
+    return lsd::host_copy(m->stage, m->stream, &out, 1, true);
 }
 
 int lsd_mlp_grad(lsd_mlp* m, long rows, const float* x, const float* target, float* loss, float* grad) {

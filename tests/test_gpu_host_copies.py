@@ -1,0 +1,36 @@
+"""Copies to and from a caller's arrays below and above the size from which
+they go through pinned chunks, with a last chunk of one element, whole chunks
+and a rest: state fields set and read back, exactly; both directions of the
+network's forward pass against slices small enough for the plain copy."""
+import numpy as np
+import pytest
+
+from lsd import make_config
+from lsd.gpu import Context, Mlp
+
+pytestmark = pytest.mark.gpu
+
+
+# H = 528 (L = 32) and 4656 (L = 96) coll rows: 2 x 8 x H N bytes a field
+@pytest.mark.parametrize("L,N", [(32, 7), (32, 31), (32, 248), (32, 249), (32, 256), (96, 127)])
+def test_state_fields(L, N):
+    cfg = make_config(L=L, M=L, N=N, dt=1e-6)
+    g = Context(cfg)
+    H = cfg.sizes()[0]
+    rng = np.random.default_rng(N)
+    want = [rng.standard_normal((2, H, N)) for _ in range(6)]
+    for k in (0, 1, 2, 4, 5):
+        g.set_coll(k, want[k][0], want[k][1])
+    for k in (0, 1, 2, 4, 5):
+        re, im = g.get_coll(k)
+        assert np.array_equal(re, want[k][0]) and np.array_equal(im, want[k][1])
+    g.close()
+
+
+@pytest.mark.parametrize("rows", [1000, 32768, 32769, 70001])
+def test_network_forward(rows):
+    net = Mlp(16, 32, 16)
+    x = np.random.default_rng(rows).standard_normal((rows, 16)).astype(np.float32)
+    y = net.forward(x)
+    for r in range(0, rows, 5000):
+        assert np.array_equal(y[r:r + 5000], net.forward(x[r:r + 5000]))
