@@ -77,19 +77,6 @@ __device__ __forceinline__ BlockId decode_block(int ngroups, int ncc) {
 }
 static unsigned grid_blocks(int ngroups, int ncc) { return (unsigned)(((ngroups + 7) / 8) * 8 * ncc); }
 
-// The value of the neighbouring lane (lane ^ 1): a DPP quad permutation
-// [1, 0, 3, 2], a register move rather than a trip through the LDS crossbar.
-constexpr int DPP_SWAP_PAIRS = 0xB1;
-__device__ __forceinline__ float partner(float v) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), DPP_SWAP_PAIRS, 0xF, 0xF, false));
-}
-__device__ __forceinline__ double partner(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, DPP_SWAP_PAIRS, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), DPP_SWAP_PAIRS, 0xF, 0xF, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
 // Up to LG_MAXJ transforms of one kind run as one launch (jobs): they read
 // the same tables, so their column chunks are placed in the same table
 // groups.
@@ -107,28 +94,20 @@ __device__ __forceinline__ P pickj(const P (&v)[LG_MAXJ], int j) {
     return r;
 }
 
-template <typename T>
 struct SynArgs {
-    int N, Th, Th2, M, MP, H;
-    int nth, ncc, nmg, njob;  // theta blocks, column blocks per job, m groups, jobs
+    int N, Th, Th2, M, MP;
+    int nth, ncc, nmg, njob;  // theta blocks, shell blocks, m groups, jobs
     const Slot* slots;
-    const int* mslot;         // [M] slot of each FFT index m
-    const T* tabA;            // [h][Th2]
-    const T* tabB;            // second table (vector / gradient)
+    const int* mslot;           // [M] slot of each FFT index m
+    const double* tabA;         // [h][Th2]
+    const double* tabB;         // second table (vector / gradient)
     const double* rinv;
-    const T* in0[LG_MAXJ];    // coll [h][2N] (re, im interleaved)
-    const T* in1[LG_MAXJ];
-    T* out0[LG_MAXJ];         // fourier [n][Th][MP] complex
-    T* out1[LG_MAXJ];
+    const double* in0[LG_MAXJ];  // coll [h][2N] (re, im interleaved)
+    const double* in1[LG_MAXJ];
+    double* out0[LG_MAXJ];       // fourier [n][Th][MP] complex
+    double* out1[LG_MAXJ];
     int out32;                // outputs rounded to FP32 (float2 Fourier layout)
 };
-
-constexpr int SY_TH = 16;     // theta points per tile (the MFMA's 16 columns)
-constexpr int SY_COLS = 16;   // coefficient columns per tile (8 shells, re/im)
-constexpr int SY_MG = 8;      // FFT indices m per workgroup
-constexpr int SY_WAVES = 4;   // waves per workgroup (SY_MG / SY_WAVES m each)
-constexpr int SY_SP = 2 * SY_MG + 1;  // LDS row of one (output, mirror, shell, theta): MG re/im pairs + pad
-constexpr int SY_PD = 4;      // K steps per prefetch group
 
 // Row (coefficient column) of accumulator element r held by lane group q4:
 // v_mfma_f32_16x16x4f32 gives rows 4 q4 + r, the FP64 instruction q4 + 4 r.
@@ -137,159 +116,201 @@ __device__ __forceinline__ int acc_row(int q4, int r) {
     return sizeof(T) == 8 ? q4 + 4 * r : 4 * q4 + r;
 }
 
-// Synthesis into the transposed Fourier layout [n][j][m].  A workgroup
-// takes one tile of 16 theta points x 16 columns for SY_MG consecutive m:
-// each wave contracts its m values one after another (KIND 0: scalar P;
-// 1: vector (llP_ flipped, llsin1mP); 2: gradient (P_ flipped, sin1mP,
-// scaled by 1/r)), with the operands of the next group of SY_PD K steps
-// loaded while the current group's products run, and leaves its results in
-// LDS; the workgroup then writes, for every (shell, theta row), the SY_MG
-// values of consecutive m as one contiguous run.
-template <typename T, int KIND>
-__global__ void __launch_bounds__(64 * SY_WAVES) k_syn(SynArgs<T> a) {
-    typedef typename Mfma<T>::acc acc_t;
-    typedef typename std::conditional<sizeof(T) == 8, double2, float2>::type T2;
+// Synthesis into the transposed Fourier layout [n][j][m] (KIND 0: scalar P;
+// 1: vector (llP_ flipped, llsin1mP); 2: gradient (P_ flipped, sin1mP, scaled
+// by 1/r)).  A wave takes one m, 16 shells and 16 TN theta:
+// * a lane's 16-byte load of a coefficient row is (re, im) of one shell, the A
+//   operands of two column tiles, so the i rotations are a swap within it;
+// * a lane's load of a table row is TN consecutive theta, the B operands of TN
+//   theta tiles (tile t holds theta TN l16 + t).
+// The operands of step k0 + 8 S8_NB (8 harmonics each) are loaded after the
+// products of step k0.  The MG waves of a workgroup take consecutive m and
+// pass their results through LDS, one (output, theta tile) at a time, so
+// each row gets them as one contiguous run.
+// Bound: a 16 x 16 tile per wave reads two or one operands per MFMA, all of
+// them from L2 (the waves of a workgroup share nothing), at 6-8 TB/s; TN = 2
+// halves that, and the rest is the store of the Fourier rows and the matrix
+// cores.  L = M = 170, N = 96, against one 16 x 16 tile and 8-byte loads:
+// vector 468 -> 293 us (156 of MFMAs), scalar 269 -> 179 us (88 of stores),
+// gradient 203 -> 123 us (59 of stores).
+constexpr int S8_SH = 16;  // shells per wave
+constexpr int S8_TH = 16;  // theta points per MFMA tile
+constexpr int S8_NB = 2;   // operand buffers
+
+// theta pairs start at any theta: 8-byte alignment only
+typedef double d2a8 __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int KIND, int TN, int MG>
+__global__ void __launch_bounds__(64 * MG) __attribute__((amdgpu_waves_per_eu(KIND == 0 ? 4 : 2)))
+k_syn8(SynArgs a) {
+    static_assert(TN == 1 || TN == 2, "one theta or a pair per lane");
     constexpr int NOUT = KIND == 0 ? 1 : 2;
-    __shared__ T St[NOUT * 2 * 8 * SY_TH * SY_SP];
-    // groups (m group, job, column block), the theta blocks of one group
+    __shared__ double2 St[2 * S8_SH * S8_TH * (MG + 1)];  // [mirror][shell][theta][m]
+    // groups (m group, job, shell block), the theta blocks of one group
     // consecutive on one XCD: they read the same coefficient rows
     const BlockId bid = decode_block(a.nmg * a.njob * a.ncc, a.nth);
     if (!bid.valid) return;
     const int mg = bid.group / (a.njob * a.ncc);
     const int gjc = bid.group - mg * a.njob * a.ncc;
-    const int job = gjc / a.ncc, cc = gjc - job * a.ncc, tb = bid.cc;
-    const int j0 = tb * SY_TH, c0 = cc * SY_COLS, m0 = mg * SY_MG;
-    const T* in0 = pickj(a.in0, job);
-    const T* in1 = pickj(a.in1, job);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, l16 = lane & 15, q4 = lane >> 4;
-    const int C2 = 2 * a.N;
-    const bool odd_col = (l16 & 1);
-    const int jc = j0 + l16 < a.Th2 ? j0 + l16 : a.Th2 - 1;
-    const int c = c0 + l16;
+    const int job = gjc / a.ncc, n0 = (gjc - job * a.ncc) * S8_SH;
+    const int j0 = bid.cc * S8_TH * TN, m0 = mg * MG;
+    const double2* in0 = reinterpret_cast<const double2*>(pickj(a.in0, job));
+    const double2* in1 = KIND == 1 ? reinterpret_cast<const double2*>(pickj(a.in1, job)) : nullptr;
+    const int tid = threadIdx.x, wave = uniform(tid >> 6), lane = tid & 63, l16 = lane & 15, q4 = lane >> 4;
+    const int nc = min(n0 + l16, a.N - 1);
+    // the second theta of a pair may lie one past the row (the table has a
+    // spare element past its last row); its results are not stored
+    const int jc = min(j0 + TN * l16, a.Th2 - 1);
     struct Ops {
-        T ta[2], tb[2], x[2], t[2];
+        double ta[2][TN], tb[2][TN];
+        double2 x[2], t[2];
     };
-#pragma unroll 1
-    for (int mi = wave; mi < SY_MG; mi += SY_WAVES) {
-        const int m = m0 + mi;
-        acc_t Y[NOUT][2];
+    v4d Y[NOUT][2][2][TN];  // [output][bucket][re, im][theta tile]
 #pragma unroll
-        for (int o = 0; o < NOUT; o++) Y[o][0] = Y[o][1] = acc_t{0, 0, 0, 0};
-        if (m < a.M) {
-            const Slot s = a.slots[a.mslot[m]];
-            auto load = [&](Ops& op, int k0) {
+    for (int o = 0; o < NOUT; o++)
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+#pragma unroll
+            for (int t = 0; t < TN; t++) Y[o][p][0][t] = Y[o][p][1][t] = v4d{0, 0, 0, 0};
+    const int m = m0 + wave;
+    if (m < a.M) {
+        const Slot s = a.slots[a.mslot[m]];
+        auto row = [&](const double* tab, size_t at, double (&v)[TN]) {
+            if constexpr (TN == 2) {
+                const d2a8 w = *reinterpret_cast<const d2a8*>(tab + at);
+                v[0] = w.x;
+                v[TN - 1] = w.y;
+            } else {
+                v[0] = tab[at];
+            }
+        };
+        auto load = [&](Ops& op, int k0) {
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const size_t h = (size_t)s.h0 + min(k0 + 2 * q4 + p, s.len - 1);
+                row(a.tabA, h * a.Th2 + jc, op.ta[p]);
+                if constexpr (KIND != 0) row(a.tabB, h * a.Th2 + jc, op.tb[p]);
+                op.x[p] = in0[h * a.N + nc];
+                if constexpr (KIND == 1) op.t[p] = in1[h * a.N + nc];
+            }
+        };
+        auto step = [&](Ops& op, int k0) {
+            if (k0 + 8 > s.len) {  // harmonics past the slot add nothing
 #pragma unroll
                 for (int p = 0; p < 2; p++) {
-                    const int k = k0 + 2 * q4 + p;
-                    const bool kv = k < s.len;
-                    const size_t hrow = (size_t)s.h0 + (kv ? k : 0);
-                    op.ta[p] = kv ? a.tabA[hrow * a.Th2 + jc] : T(0);
-                    op.tb[p] = (KIND != 0 && kv) ? a.tabB[hrow * a.Th2 + jc] : T(0);
-                    const bool cv = kv && c < C2;
-                    op.x[p] = cv ? in0[hrow * C2 + c] : T(0);
-                    op.t[p] = (KIND == 1 && cv) ? in1[hrow * C2 + c] : T(0);
-                }
-            };
-            auto step = [&](const Ops& op) {
-#pragma unroll
-                for (int p = 0; p < 2; p++) {
-                    const T x = op.x[p];
-                    if (KIND == 0) {
-                        Y[0][p] = Mfma<T>::run(x, op.ta[p], Y[0][p]);
-                    } else if (KIND == 2) {
-                        // theta: c * dP (bucket 1-p);  phi: (i c) * mP/sin (bucket p)
-                        T xr = partner(x);
-                        xr = odd_col ? xr : -xr;
-                        Y[0][1 - p] = Mfma<T>::run(x, op.ta[p], Y[0][1 - p]);
-                        Y[NOUT - 1][p] = Mfma<T>::run(xr, op.tb[p], Y[NOUT - 1][p]);
-                    } else {
-                        const T t = op.t[p];
-                        // (-i t): re <- t_im, im <- -t_re ;  (i s): re <- -s_im, im <- s_re
-                        T tr = partner(t), sr = partner(x);
-                        tr = odd_col ? -tr : tr;
-                        sr = odd_col ? sr : -sr;
-                        Y[0][1 - p] = Mfma<T>::run(x, op.ta[p], Y[0][1 - p]);
-                        Y[0][p] = Mfma<T>::run(tr, op.tb[p], Y[0][p]);
-                        Y[NOUT - 1][p] = Mfma<T>::run(sr, op.tb[p], Y[NOUT - 1][p]);
-                        Y[NOUT - 1][1 - p] = Mfma<T>::run(t, op.ta[p], Y[NOUT - 1][1 - p]);
+                    const bool kv = k0 + 2 * q4 + p < s.len;
+                    op.x[p].x = kv ? op.x[p].x : 0.0;
+                    op.x[p].y = kv ? op.x[p].y : 0.0;
+                    if constexpr (KIND == 1) {
+                        op.t[p].x = kv ? op.t[p].x : 0.0;
+                        op.t[p].y = kv ? op.t[p].y : 0.0;
                     }
                 }
-            };
-            // groups of SY_PD steps (8 harmonics each), two groups in flight
-            Ops ga[SY_PD], gb[SY_PD];
+            }
 #pragma unroll
-            for (int u = 0; u < SY_PD; u++) load(ga[u], 8 * u);
-            for (int k0 = 0; k0 < s.len; k0 += 16 * SY_PD) {
-                const int k1 = k0 + 8 * SY_PD;
-                if (k1 < s.len) {
+            for (int p = 0; p < 2; p++) {
+                const double2 x = op.x[p];
 #pragma unroll
-                    for (int u = 0; u < SY_PD; u++) load(gb[u], k1 + 8 * u);
+                for (int t = 0; t < TN; t++) {
+                    const double ta = op.ta[p][t];
+                    if constexpr (KIND == 0) {
+                        Y[0][p][0][t] = Mfma<double>::run(x.x, ta, Y[0][p][0][t]);
+                        Y[0][p][1][t] = Mfma<double>::run(x.y, ta, Y[0][p][1][t]);
+                    } else if constexpr (KIND == 2) {
+                        // theta: c * dP (bucket 1-p);  phi: (i c) * mP/sin (bucket p)
+                        const double tb = op.tb[p][t];
+                        Y[0][1 - p][0][t] = Mfma<double>::run(x.x, ta, Y[0][1 - p][0][t]);
+                        Y[0][1 - p][1][t] = Mfma<double>::run(x.y, ta, Y[0][1 - p][1][t]);
+                        Y[NOUT - 1][p][0][t] = Mfma<double>::run(-x.y, tb, Y[NOUT - 1][p][0][t]);
+                        Y[NOUT - 1][p][1][t] = Mfma<double>::run(x.x, tb, Y[NOUT - 1][p][1][t]);
+                    } else {
+                        // theta: s (bucket 1-p) - i t (bucket p);  phi: i s (bucket p) + t (bucket 1-p)
+                        const double tb = op.tb[p][t];
+                        const double2 w = op.t[p];
+                        Y[0][1 - p][0][t] = Mfma<double>::run(x.x, ta, Y[0][1 - p][0][t]);
+                        Y[0][1 - p][1][t] = Mfma<double>::run(x.y, ta, Y[0][1 - p][1][t]);
+                        Y[0][p][0][t] = Mfma<double>::run(w.y, tb, Y[0][p][0][t]);
+                        Y[0][p][1][t] = Mfma<double>::run(-w.x, tb, Y[0][p][1][t]);
+                        Y[NOUT - 1][p][0][t] = Mfma<double>::run(-x.y, tb, Y[NOUT - 1][p][0][t]);
+                        Y[NOUT - 1][p][1][t] = Mfma<double>::run(x.x, tb, Y[NOUT - 1][p][1][t]);
+                        Y[NOUT - 1][1 - p][0][t] = Mfma<double>::run(w.x, ta, Y[NOUT - 1][1 - p][0][t]);
+                        Y[NOUT - 1][1 - p][1][t] = Mfma<double>::run(w.y, ta, Y[NOUT - 1][1 - p][1][t]);
+                    }
                 }
+            }
+        };
+        Ops ops[S8_NB];
 #pragma unroll
-                for (int u = 0; u < SY_PD; u++)
-                    if (k0 + 8 * u < s.len) step(ga[u]);
-                if (k1 >= s.len) break;
-                if (k1 + 8 * SY_PD < s.len) {
+        for (int u = 0; u < S8_NB; u++) load(ops[u], 8 * u);
+        for (int k0 = 0; k0 < s.len; k0 += 8 * S8_NB) {
 #pragma unroll
-                    for (int u = 0; u < SY_PD; u++) load(ga[u], k1 + 8 * SY_PD + 8 * u);
-                }
-#pragma unroll
-                for (int u = 0; u < SY_PD; u++)
-                    if (k1 + 8 * u < s.len) step(gb[u]);
+            for (int u = 0; u < S8_NB; u++) {
+                if (k0 + 8 * u < s.len) step(ops[u], k0 + 8 * u);
+                load(ops[u], k0 + 8 * (u + S8_NB));
             }
         }
-        // F[j] = Y0 + Y1, F[Th-1-j] = Y0 - Y1; lane: theta l16, rows acc_row
+    }
+    // F[j] = Y0 + Y1, F[Th-1-j] = Y0 - Y1; lane: theta l16 of the tile, shells
+    // acc_row
 #pragma unroll
-        for (int o = 0; o < NOUT; o++)
+    for (int o = 0; o < NOUT; o++)
+#pragma unroll
+        for (int t = 0; t < TN; t++) {
+            if (o + t > 0) __syncthreads();
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int row = acc_row<T>(q4, r), sh = row >> 1, part = row & 1;
-                const T y0 = Y[o][0][r], y1 = Y[o][1][r];
-                T* d = St + (((o * 2 + 0) * 8 + sh) * SY_TH + l16) * SY_SP + 2 * mi + part;
-                d[0] = y0 + y1;
-                d[8 * SY_TH * SY_SP] = y0 - y1;
+                double2* d = St + (acc_row<double>(q4, r) * S8_TH + l16) * (MG + 1) + wave;
+                const double re0 = Y[o][0][0][t][r], re1 = Y[o][1][0][t][r];
+                const double im0 = Y[o][0][1][t][r], im1 = Y[o][1][1][t][r];
+                d[0] = make_double2(re0 + re1, im0 + im1);
+                d[S8_SH * S8_TH * (MG + 1)] = make_double2(re0 - re1, im0 - im1);
             }
-    }
-    __syncthreads();
-    constexpr int NITEM = NOUT * 2 * 8 * SY_TH * SY_MG;
-    for (int idx = tid; idx < NITEM; idx += 64 * SY_WAVES) {
-        const int mi = idx % SY_MG;
-        int rest = idx / SY_MG;
-        const int th = rest % SY_TH;
-        rest /= SY_TH;
-        const int sh = rest % 8;
-        rest /= 8;
-        const int mir = rest & 1, o = rest >> 1;
-        const int n = (c0 >> 1) + sh, j = j0 + th;
-        if (n >= a.N || j >= a.Th2) continue;
-        const int jrow = mir ? a.Th - 1 - j : j;
-        if (mir && jrow < a.Th2) continue;
-        const T* sp = St + (((o * 2 + mir) * 8 + sh) * SY_TH + th) * SY_SP + 2 * mi;
-        const T f = KIND == 2 ? (T)a.rinv[n] : T(1);
-        T2 v;
-        v.x = f * sp[0];
-        v.y = f * sp[1];
-        T* out = o == 0 ? pickj(a.out0, job) : pickj(a.out1, job);
-        const size_t at = ((size_t)n * a.Th + jrow) * a.MP + m0 + mi;
-        if (a.out32) reinterpret_cast<float2*>(out)[at] = make_float2((float)v.x, (float)v.y);
-        else reinterpret_cast<T2*>(out)[at] = v;
-    }
+            __syncthreads();
+            double* out = o == 0 ? pickj(a.out0, job) : pickj(a.out1, job);
+#pragma unroll
+            for (int it = 0; it < 2 * S8_SH * S8_TH / 64; it++) {
+                const int idx = tid + 64 * MG * it;
+                const int mi = idx % MG, th = idx / MG % S8_TH, sh = idx / (MG * S8_TH) % S8_SH;
+                const int mir = idx / (MG * S8_TH * S8_SH);
+                const int n = n0 + sh, j = j0 + TN * th + t;
+                if (n >= a.N || j >= a.Th2) continue;
+                const int jrow = mir ? a.Th - 1 - j : j;
+                if (mir && jrow < a.Th2) continue;
+                double2 v = St[((mir * S8_SH + sh) * S8_TH + th) * (MG + 1) + mi];
+                if constexpr (KIND == 2) {
+                    const double f = a.rinv[n];
+                    v.x = f * v.x;
+                    v.y = f * v.y;
+                }
+                const size_t at = ((size_t)n * a.Th + jrow) * a.MP + m0 + mi;
+                if (a.out32) reinterpret_cast<float2*>(out)[at] = make_float2((float)v.x, (float)v.y);
+                else reinterpret_cast<double2*>(out)[at] = v;
+            }
+        }
 }
 
-template <typename T>
-static int syn_launch(Ctx& c, int kind, int njob, const T* tA, const T* tB, const void* const* in0,
-                      const void* const* in1, void* const* out0, void* const* out1, bool out32 = false) {
+template <int TN, int MG>
+static void syn8_launch(Ctx& c, int kind, SynArgs& a) {
+    a.nth = (c.Th2 + S8_TH * TN - 1) / (S8_TH * TN);
+    a.nmg = (c.M + MG - 1) / MG;
+    const dim3 grid(grid_blocks(a.nmg * a.njob * a.ncc, a.nth)), blk(64 * MG);
+    if (kind == SYN_SCALAR) hipLaunchKernelGGL((k_syn8<0, TN, MG>), grid, blk, 0, c.stream, a);
+    else if (kind == SYN_VECTOR) hipLaunchKernelGGL((k_syn8<1, TN, MG>), grid, blk, 0, c.stream, a);
+    else hipLaunchKernelGGL((k_syn8<2, TN, MG>), grid, blk, 0, c.stream, a);
+}
+
+static int syn_launch(Ctx& c, int kind, int njob, const double* tA, const double* tB, const void* const* in0,
+                      const void* const* in1, void* const* out0, void* const* out1, bool out32) {
     if (njob < 1 || njob > LG_MAXJ) {
         set_error("synthesis: 1..6 transforms per launch");
         return LSD_E_ARG;
     }
-    SynArgs<T> a;
+    SynArgs a;
     a.N = c.N;
     a.Th = c.Th;
     a.Th2 = c.Th2;
     a.M = c.M;
     a.MP = c.MP;
-    a.H = c.H;
     a.slots = c.d_slots;
     a.mslot = c.d_mslot;
     a.tabA = tA;
@@ -298,20 +319,22 @@ static int syn_launch(Ctx& c, int kind, int njob, const T* tA, const T* tB, cons
     a.out32 = out32 ? 1 : 0;
     for (int k = 0; k < LG_MAXJ; k++) {
         const int q = k < njob ? k : 0;
-        a.in0[k] = reinterpret_cast<const T*>(in0[q]);
-        a.in1[k] = in1 ? reinterpret_cast<const T*>(in1[q]) : nullptr;
-        a.out0[k] = reinterpret_cast<T*>(out0[q]);
-        a.out1[k] = out1 ? reinterpret_cast<T*>(out1[q]) : nullptr;
+        a.in0[k] = reinterpret_cast<const double*>(in0[q]);
+        a.in1[k] = in1 ? reinterpret_cast<const double*>(in1[q]) : nullptr;
+        a.out0[k] = reinterpret_cast<double*>(out0[q]);
+        a.out1[k] = out1 ? reinterpret_cast<double*>(out1[q]) : nullptr;
     }
-    a.nth = (c.Th2 + SY_TH - 1) / SY_TH;
-    a.ncc = (2 * c.N + SY_COLS - 1) / SY_COLS;
-    a.nmg = (c.M + SY_MG - 1) / SY_MG;
+    a.ncc = (c.N + S8_SH - 1) / S8_SH;
     a.njob = njob;
-    dim3 grid(grid_blocks(a.nmg * njob * a.ncc, a.nth));
-    dim3 blk(64 * SY_WAVES);
-    if (kind == SYN_SCALAR) hipLaunchKernelGGL((k_syn<T, 0>), grid, blk, 0, c.stream, a);
-    else if (kind == SYN_VECTOR) hipLaunchKernelGGL((k_syn<T, 1>), grid, blk, 0, c.stream, a);
-    else hipLaunchKernelGGL((k_syn<T, 2>), grid, blk, 0, c.stream, a);
+    // Theta pairs and eight m per workgroup where that still gives every CU a
+    // workgroup; smaller launches need the parallelism more.  Vector kind, pairs
+    // and eight m against one theta and four: 17.3 and 9.1 us with 32 and 128
+    // workgroups (L = M = 32, N = 32), 25.6 and 11.4 us with 64 and 192
+    // (L = M = 64, N = 64, one field), 293 and 361 us with 2112 and 8448
+    // (L = M = 170, N = 96).
+    const long big = (long)((c.M + 7) / 8) * njob * a.ncc * ((c.Th2 + 2 * S8_TH - 1) / (2 * S8_TH));
+    if (big >= c.ncu) syn8_launch<2, 8>(c, kind, a);
+    else syn8_launch<1, 4>(c, kind, a);
     LSD_HIP(hipGetLastError());
     return LSD_OK;
 }
@@ -344,7 +367,7 @@ int launch_synthesis_group(Ctx& c, int kind, int njob, const void* const* in0, c
         const size_t p1 = (kind == SYN_VECTOR ? 4 : 2) * HTp;
         return syn4_launch(c, kind, njob, c.d_tab32 + p0, c.d_tab32 + p1, in0, in1, out0, out1);
     }
-    return syn_launch<double>(c, kind, njob, c.d_tab + o0, c.d_tab + o1, in0, in1, out0, out1, out32);
+    return syn_launch(c, kind, njob, c.d_tab + o0, c.d_tab + o1, in0, in1, out0, out1, out32);
 }
 
 int launch_synthesis_p(Ctx& c, int kind, const void* in0, const void* in1, void* out0, void* out1, bool f32) {

@@ -271,7 +271,7 @@ static int create(const lsd_config* cfg, int device, Ctx** out) {
         dalloc(&c->d_apos, H) || dalloc(&c->d_slots, c->nslot) || dalloc(&c->d_slot_order, c->nslot) ||
         dalloc(&c->d_mslot, c->M) ||
         dalloc(&c->d_gp, Th) || dalloc(&c->d_gw, Th) || dalloc(&c->d_sin, Th) ||
-        dalloc(&c->d_tab, (size_t)5 * H * c->Th2) || dalloc(&c->d_atab, (size_t)3 * H * c->Th2) ||
+        dalloc(&c->d_tab, (size_t)5 * H * c->Th2 + 1) || dalloc(&c->d_atab, (size_t)3 * H * c->Th2) ||
         dalloc(&c->d_r, (size_t)7 * N) || dalloc(&c->d_dr1, (size_t)7 * N) || dalloc(&c->d_dr2, (size_t)7 * N) ||
         dalloc(&c->d_radlap, (size_t)7 * N) || dalloc(&c->d_r1dr, (size_t)7 * N) || dalloc(&c->d_intr2dr, N) ||
         dalloc(&c->d_ll, (size_t)4 * L) || dalloc(&c->d_lu, (size_t)NLU * L * N * LSD_LDAB) ||
@@ -402,7 +402,7 @@ static int create(const lsd_config* cfg, int device, Ctx** out) {
         LSD_HIP(hipMemcpyAsync(c->d_mslot, mslot.data(), sizeof(int) * c->M, hipMemcpyHostToDevice, st));
         LSD_HIP(hipStreamSynchronize(st));
     }
-    LSD_HIP(hipMemsetAsync(c->d_tab, 0, sizeof(double) * 5 * H * c->Th2, st));
+    LSD_HIP(hipMemsetAsync(c->d_tab, 0, sizeof(double) * ((size_t)5 * H * c->Th2 + 1), st));
     LSD_HIP(hipMemsetAsync(c->d_atab, 0, sizeof(double) * 3 * H * c->Th2, st));
     LSD_HIP(hipMemsetAsync(c->d_lu, 0, sizeof(double) * NLU * L * N * LSD_LDAB, st));
     LSD_HIP(hipMemsetAsync(c->d_piv, 0, sizeof(int) * NLU * L * N, st));
