@@ -14,7 +14,7 @@ runs the same number of steps by graph replay for the ratio.  The per-field
 relative error of the mixed form against the plain FP64 form is measured
 after 1 and after 1000 steps from the same seeded state.  ``roofline``
 reports the largest single kernel of the mixed step, the fused
-physical-space pass (k_physfuse: phi FFTs, products and the equatorial
+physical-space pass (k_physwave: phi FFTs, products and the equatorial
 fold), timed with HIP events on the context's stream in a separate eager
 run of the same steps; ``traffic`` is its HBM bytes per launch from the
 rocprofv3 FETCH_SIZE / WRITE_SIZE counters recorded in
@@ -277,7 +277,7 @@ def main():
     achieved = per_launch / avg_s / 1e9
     roof = {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": achieved / PEAK_HBM_GBS}
-    roof["kernel"] = "k_physfuse (class %s)" % K_NAMES[dom]
+    roof["kernel"] = "k_physwave (class %s)" % K_NAMES[dom]
     roof["algorithmic_bytes_per_launch"] = per_launch
     roof["launches"] = nl
     roof["avg_launch_ms"] = avg_s * 1e3

@@ -561,43 +561,53 @@ __global__ void k_operators(int L, int N, OpParams op, const double* __restrict_
 }
 
 // Green's functions and the 2x2 influence matrix of the poloidal velocity
-// (modules/velocity.F90:134-168), one work-item per degree l >= 1.
-__global__ void k_green(int L, int N, const double* __restrict__ lu, const int* __restrict__ piv,
-                        double* __restrict__ gre, double* __restrict__ invg, int* __restrict__ info,
-                        double* __restrict__ scratch) {
-    int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l < 1 || l >= L) return;
-    double* re = scratch + (size_t)l * 2 * N;
-    double* im = re + N;
-    for (int n = 0; n < N; n++) {
-        re[n] = 0.0;
-        im[n] = 0.0;
+// (modules/velocity.F90:134-168), one wave per degree l >= 1: the factors of
+// one kind at a time in LDS, the two right-hand sides on lanes 0 and 1.
+// Bound by the serial chain of four sweeps, a row at a time, so by the latency
+// of its operands.  A thread per degree with everything in global memory took
+// 680 us at L = 64, N = 64; with the operands in LDS the first pass of the
+// Christensen benchmark, 40 changes of dt, goes from 78 to 54 ms.
+static size_t green_lds(int N) { return (size_t)N * (sizeof(double) * (LSD_LDAB + 2) + sizeof(int)); }
+
+__global__ void __launch_bounds__(64) k_green(int L, int N, const double* __restrict__ lu,
+                                              const int* __restrict__ piv, double* __restrict__ gre,
+                                              double* __restrict__ invg, int* __restrict__ info) {
+    extern __shared__ double gsm[];
+    double* ab = gsm;                      // [N][LDAB]
+    double* cols = ab + N * LSD_LDAB;      // [2][N]
+    int* pv = reinterpret_cast<int*>(cols + 2 * N);
+    const int l = blockIdx.x + 1, t = threadIdx.x;
+    auto stage = [&](int kind) {
+        const double* src = lu + ((size_t)kind * L + l) * N * LSD_LDAB;
+        const int* ps = piv + ((size_t)kind * L + l) * N;
+        for (int i = t; i < N * LSD_LDAB; i += 64) ab[i] = src[i];
+        for (int i = t; i < N; i += 64) pv[i] = ps[i];
+    };
+    for (int i = t; i < 2 * N; i += 64) cols[i] = (i == 0 || i == 2 * N - 1) ? 1.0 : 0.0;
+    stage(2);
+    __syncthreads();
+    if (t < 2) {
+        gbtrs_d(N, ab, pv, cols + t * N);
+        cols[t * N] = cols[t * N + N - 1] = 0.0;
     }
-    re[0] = 1.0;
-    im[N - 1] = 1.0;
-    const double* abg = lu + ((size_t)2 * L + l) * N * LSD_LDAB;
-    const int* pg = piv + ((size_t)2 * L + l) * N;
-    gbtrs_d(N, abg, pg, re);
-    gbtrs_d(N, abg, pg, im);
-    re[0] = re[N - 1] = im[0] = im[N - 1] = 0.0;
-    const double* abp = lu + ((size_t)1 * L + l) * N * LSD_LDAB;
-    const int* pp = piv + ((size_t)1 * L + l) * N;
-    gbtrs_d(N, abp, pp, re);
-    gbtrs_d(N, abp, pp, im);
-    for (int n = 0; n < N; n++) {
-        gre[((size_t)l * 2 + 0) * N + n] = re[n];
-        gre[((size_t)l * 2 + 1) * N + n] = im[n];
+    __syncthreads();
+    stage(1);
+    __syncthreads();
+    if (t < 2) gbtrs_d(N, ab, pv, cols + t * N);
+    __syncthreads();
+    for (int i = t; i < 2 * N; i += 64) gre[(size_t)l * 2 * N + i] = cols[i];
+    if (t == 0) {
+        double g[14];
+        g[0] = cols[0];
+        g[1] = cols[N - 1];
+        g[7] = cols[N];
+        g[8] = cols[2 * N - 1];
+        if (invert7(2, g)) info[l] = 1;
+        invg[l * 4 + 0] = g[0];
+        invg[l * 4 + 1] = g[1];
+        invg[l * 4 + 2] = g[7];
+        invg[l * 4 + 3] = g[8];
     }
-    double g[14];
-    g[0] = re[0];
-    g[1] = re[N - 1];
-    g[7] = im[0];
-    g[8] = im[N - 1];
-    if (invert7(2, g)) info[l] = 1;
-    invg[l * 4 + 0] = g[0];
-    invg[l * 4 + 1] = g[1];
-    invg[l * 4 + 2] = g[7];
-    invg[l * 4 + 3] = g[8];
 }
 
 __global__ void k_to_f32(size_t n, const double* __restrict__ a, float* __restrict__ b) {
@@ -841,14 +851,13 @@ int build_operators(Ctx& c) {
     hipLaunchKernelGGL(k_operators, grid, dim3(64), 0, c.stream, L, N, op, c.d_r, c.d_radlap, c.d_dr1, c.d_dr2,
                        c.d_lu, c.d_piv, c.d_y, c.d_info, c.d_xband);
     LSD_HIP(hipGetLastError());
-    double* scratch = nullptr;
     int* ginfo = nullptr;
-    AsyncScratch s_scr(c.stream), s_ginfo(c.stream);
-    LSD_HIP(s_scr.alloc(&scratch, sizeof(double) * 2 * N * L));
+    AsyncScratch s_ginfo(c.stream);
     LSD_HIP(s_ginfo.alloc(&ginfo, sizeof(int) * L));
     LSD_HIP(hipMemsetAsync(ginfo, 0, sizeof(int) * L, c.stream));
-    hipLaunchKernelGGL(k_green, dim3((L + 63) / 64), dim3(64), 0, c.stream, L, N, c.d_lu, c.d_piv, c.d_gre,
-                       c.d_invg, ginfo, scratch);
+    if (L > 1)
+        hipLaunchKernelGGL(k_green, dim3(L - 1), dim3(64), green_lds(N), c.stream, L, N, c.d_lu, c.d_piv, c.d_gre,
+                           c.d_invg, ginfo);
     LSD_HIP(hipGetLastError());
     int rc_ic = build_ic_operators(c);
     if (rc_ic) return rc_ic;
