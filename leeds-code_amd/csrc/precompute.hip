@@ -466,23 +466,27 @@ struct OpParams {
     int vel_bc;  // i_vel_bc: 1 no-slip, 2 stress-free outer, 3 stress-free inner, 4 both stress-free
 };
 
-// One work-item per (operator kind, degree l): X = c1/dt - c2 c radLap_l
+// One wave per (operator kind, degree l): X = c1/dt - c2 c radLap_l
 // with boundary rows (modules/timestep.F90:138-211, 218-344;
 // velocity.F90:177-273; codensity.F90:85-119; composition.F90:82-105;
 // magnetic.F90:137-282), factorised in place, plus the explicit operator
-// Y = c1/dt + c2 (1-c) radLap_l (timestep.F90:421-473).
-__global__ void k_operators(int L, int N, OpParams op, const double* __restrict__ r,
+// Y = c1/dt + c2 (1-c) radLap_l (timestep.F90:421-473).  The lanes form and
+// copy the columns, lane 0 factorises the band in LDS: bound by that serial
+// chain, so by the latency of its operands: 121 us at L = 64, N = 64, 381 us
+// with a thread per degree and the band in global memory.
+static size_t operators_lds(int N) { return (size_t)N * (sizeof(double) * LSD_LDAB + sizeof(int)); }
+
+__global__ void __launch_bounds__(64) k_operators(int L, int N, OpParams op, const double* __restrict__ r,
                             const double* __restrict__ radlap, const double* __restrict__ dr1,
                             const double* __restrict__ dr2, double* __restrict__ lu, int* __restrict__ piv, double* __restrict__ ym,
                             int* __restrict__ info, double* __restrict__ xband) {
-    int l = blockIdx.x * blockDim.x + threadIdx.x;
-    int kind = blockIdx.y;
-    if (l >= L) return;
+    extern __shared__ double osm[];
+    double* ab = osm;  // [N][LDAB]
+    int* pv = reinterpret_cast<int*>(ab + N * LSD_LDAB);
+    const int l = blockIdx.x, kind = blockIdx.y, t = threadIdx.x;
     bool need = (kind == 3 || kind == 4) ? true : (l >= 1);
-    double* ab = lu + ((size_t)kind * L + l) * N * LSD_LDAB;
-    int* pv = piv + ((size_t)kind * L + l) * N;
     if (!need) {
-        info[kind * L + l] = 0;
+        if (t == 0) info[kind * L + l] = 0;
         return;
     }
     double c1, c2;
@@ -501,13 +505,15 @@ __global__ void k_operators(int L, int N, OpParams op, const double* __restrict_
     double ll1 = (double)(l * (l + 1));
     const double* rm2 = r + 1 * N;
     const double* rm1 = r + 2 * N;
-    for (int j = 0; j < N; j++) {
+    for (int j = t; j < N; j += 64) {
         for (int q = 0; q < LSD_KL; q++) ab[j * LSD_LDAB + q] = 0.0;
         for (int q = 0; q < 7; q++) ab[j * LSD_LDAB + LSD_KL + q] = -c2_ * radlap[j * 7 + q];
         double* d = &ab[j * LSD_LDAB + 2 * LSD_KL];
         if (diagform == 0) *d = (*d + c1_) + c2_ * (ll1 * rm2[j]);
         else *d = (*d + c1_) + c2_ * ll1 * rm2[j];
     }
+    __syncthreads();
+    if (t == 0) {
 #define LUA(i, j) ab[((j) - 1) * LSD_LDAB + (2 * LSD_KL + (i) - (j))]
 #define DR1(i, j) dr1[((j) - 1) * 7 + (LSD_KL + (i) - (j))]
 #define DR2(i, j) dr2[((j) - 1) * 7 + (LSD_KL + (i) - (j))]
@@ -540,20 +546,27 @@ __global__ void k_operators(int L, int N, OpParams op, const double* __restrict_
         LUA(1, 1) = 1.0;
         LUA(N, N) = 1.0;
     }
+    }
 #undef LUA
 #undef DR1
 #undef DR2
     // keep X itself (7 bands per column) for residuals of the mixed forms
     double* xb = xband + ((size_t)kind * L + l) * N * 7;
-    for (int j = 0; j < N; j++)
-        for (int q = 0; q < 7; q++) xb[j * 7 + q] = ab[j * LSD_LDAB + LSD_KL + q];
-    info[kind * L + l] = gbtrf_d(N, ab, pv);
+    __syncthreads();
+    for (int i = t; i < N * 7; i += 64) xb[i] = ab[i / 7 * LSD_LDAB + LSD_KL + i % 7];
+    __syncthreads();
+    if (t == 0) info[kind * L + l] = gbtrf_d(N, ab, pv);
+    __syncthreads();
+    double* abo = lu + ((size_t)kind * L + l) * N * LSD_LDAB;
+    int* pvo = piv + ((size_t)kind * L + l) * N;
+    for (int i = t; i < N * LSD_LDAB; i += 64) abo[i] = ab[i];
+    for (int i = t; i < N; i += 64) pvo[i] = pv[i];
     // explicit operator Y
     int yk = kind < 2 ? kind : (kind == 2 ? -1 : kind - 1);
     if (yk < 0) return;
     double* y = ym + ((size_t)yk * L + l) * N * 7;
     double c2y = c2 * (1.0 - op.implicit);
-    for (int j = 0; j < N; j++) {
+    for (int j = t; j < N; j += 64) {
         for (int q = 0; q < 7; q++) y[j * 7 + q] = c2y * radlap[j * 7 + q];
         double* d = &y[j * 7 + LSD_KL];
         *d = (*d + c1_) - c2y * (ll1 * rm2[j]);
@@ -565,8 +578,7 @@ __global__ void k_operators(int L, int N, OpParams op, const double* __restrict_
 // one kind at a time in LDS, the two right-hand sides on lanes 0 and 1.
 // Bound by the serial chain of four sweeps, a row at a time, so by the latency
 // of its operands.  A thread per degree with everything in global memory took
-// 680 us at L = 64, N = 64; with the operands in LDS the first pass of the
-// Christensen benchmark, 40 changes of dt, goes from 78 to 54 ms.
+// 680 us at L = 64, N = 64; with the operands in LDS it is 95 us.
 static size_t green_lds(int N) { return (size_t)N * (sizeof(double) * (LSD_LDAB + 2) + sizeof(int)); }
 
 __global__ void __launch_bounds__(64) k_green(int L, int N, const double* __restrict__ lu,
@@ -847,9 +859,8 @@ int build_ic_operators(Ctx& c) {
 int build_operators(Ctx& c) {
     OpParams op{c.dt, c.cfg.implicit, c.cfg.Pm, c.cfg.Pr, c.cfg.Sc, c.cfg.vel_bc};
     int L = c.L, N = c.N;
-    dim3 grid((L + 63) / 64, NLU);
-    hipLaunchKernelGGL(k_operators, grid, dim3(64), 0, c.stream, L, N, op, c.d_r, c.d_radlap, c.d_dr1, c.d_dr2,
-                       c.d_lu, c.d_piv, c.d_y, c.d_info, c.d_xband);
+    hipLaunchKernelGGL(k_operators, dim3(L, NLU), dim3(64), operators_lds(N), c.stream, L, N, op, c.d_r, c.d_radlap,
+                       c.d_dr1, c.d_dr2, c.d_lu, c.d_piv, c.d_y, c.d_info, c.d_xband);
     LSD_HIP(hipGetLastError());
     int* ginfo = nullptr;
     AsyncScratch s_ginfo(c.stream);
