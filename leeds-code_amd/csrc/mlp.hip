@@ -288,7 +288,9 @@ __global__ void __launch_bounds__(64 * MF_WAVES) k_mlp_fwd(MlpArgs g) {
                         Z[row * g.width + j] = z;
                         H[row * g.width + j] = h;
                     }
-                    So[row * MF_LD + j] = (__bf16)h;
+                    // zero past the width, also where the row holds an
+                    // infinity: it would meet the zero weights there as NaN
+                    So[row * MF_LD + j] = (__bf16)(in ? h : 0.f);
                 }
         }
         __syncthreads();

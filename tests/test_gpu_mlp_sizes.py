@@ -41,3 +41,21 @@ def test_sizes(n_in, width, n_out, rows):
     part = [m.grad(X[:batch], T[:batch])[0], m.grad(X[batch:], T[batch:])[0] if rows > batch else m.grad(X, T)[0]]
     assert np.array_equal(losses, np.array(part, dtype=np.float32))
     m.close()
+
+
+@pytest.mark.parametrize("width", [1, 16, 63, 64, 100, 250])
+def test_infinite_inputs(width):
+    """A row with an infinite input gives what the layers' definition gives:
+    with positive weights +inf, not the NaN of an infinity times the zeros
+    that pad the width; the other rows keep their results."""
+    m = Mlp(4, width, 3, seed=1)
+    m.set_params(np.full(m.n_params, 0.125, dtype=np.float32))
+    X = np.random.default_rng(2).standard_normal((40, 4)).astype(np.float32)
+    want = m.forward(X)
+    X[[5, 39], 2] = np.inf
+    y = m.forward(X)
+    assert np.all(y[[5, 39]] == np.inf)
+    rest = np.ones(40, dtype=bool)
+    rest[[5, 39]] = False
+    assert np.array_equal(y[rest], want[rest])
+    m.close()
