@@ -34,13 +34,26 @@ namespace lsd {
 // Threads per workgroup: one per phi point, the least of 64, 128, 256, 512
 // and 1024 that is not below Ph: idle waves still meet every barrier (FP64,
 // 64 shells of 96 x 48: 197 us per launch with 512 threads, 41 us with 64;
-// 32 shells of 48 x 96: 55 us with 512, 25 us with 128).
+// 32 shells of 48 x 96: 55 us with 512, 25 us with 128).  Twice as many up to
+// Ph = 128 where that fills more than half of them and a CU gets one workgroup
+// at most: the waves do not compete yet, and a thread has half the butterflies
+// of a stage (8 shells of 56 x 108, FP32 / FP64: 26 / 28 us with 128 threads,
+// 22 / 24 us with 256, 23 / 25 us with 512; of 28 x 54: 24 / 26 us with 64, 21 /
+// 23 with 128, 22 / 24 with 512).  Elsewhere the fitted count is as fast or
+// faster (8 shells of 72 x 144: 28 us, 32 with twice as many; 40 shells of 20
+// x 32 in FP64: 17 and 20 us).
 constexpr int PF_THREADS = 512;
 constexpr int PF_THREADS_MAX = 1024;
+constexpr int PF_DOUBLE_MAX = 128;
 static int pf_threads(int Ph) {
     int nt = 64;
     while (nt < Ph && nt < PF_THREADS_MAX) nt *= 2;
     return nt;
+}
+static int pf_launch_threads(const Ctx& c) {
+    const int nt = pf_threads(c.Ph);
+    const bool few = c.Ph <= PF_DOUBLE_MAX && 2 * c.Ph > nt && (long)c.N * c.Th2 <= c.ncu;
+    return few ? 2 * nt : nt;
 }
 constexpr int PF_EPT = 8;      // 8 sequences x 512 points = one radix-8 butterfly per thread
 constexpr int PF_MAXSEQ = 8;
@@ -576,7 +589,8 @@ bool physfuse_supported(const Ctx& c) {
     return c.Ph <= PF_THREADS_MAX && c.Th % 2 == 0 && 6 * c.M <= PF_ITEMS * pf_threads(c.Ph);
 }
 
-// The wave form (physwave.h); 1: a length it is not instantiated for.
+// The wave form (physwave.h); 1: a length it is not instantiated for, or a
+// launch too small for it.
 static int physwave_launch(Ctx& c, const PhysArgs<float>& a) {
     PwArgs<float> w;
     w.N = a.N;
@@ -643,7 +657,8 @@ static int physfuse_launch(Ctx& c, const void* fourier, void* folded, const void
     a.ePm = (R)k.Pm;
     if (c.cfl_on) c.cfl_parts = c.Th2;
     // FP32 takes the wave form at the lengths it is instantiated for, where
-    // the 3/2 rule leaves the upper third of the orders empty.  FP64 keeps
+    // the 3/2 rule leaves the upper third of the orders empty and the launch
+    // is large enough for it (physwave_pays).  FP64 keeps
     // this form and its rounding: plain runs go on bit for bit from recorded
     // states (the wave form in FP64 measured 31 against 55 us at 48 x 96, 32
     // shells and 535 against 640 us at 256 x 512, 96 shells, but chaotic runs
@@ -681,7 +696,7 @@ static int physfuse_launch(Ctx& c, const void* fourier, void* folded, const void
         if (c.cfl_on) PF_RUN(true, PF_THREADS, true, false);
         else PF_RUN(true, PF_THREADS, false, false);
     } else {
-        switch (pf_threads(c.Ph)) {
+        switch (pf_launch_threads(c)) {
         case 64: PF_RUN_NT(64); break;
         case 128: PF_RUN_NT(128); break;
         case 256: PF_RUN_NT(256); break;

@@ -624,9 +624,31 @@ __global__ void __launch_bounds__(64 * PL::W) __attribute__((amdgpu_waves_per_eu
     }
 }
 
+// Whether the wave form is the faster one for this launch.  Its time is one
+// row pair's chain of stages per round, a round being the row pairs that the
+// registers and the LDS of all CUs hold, whether the round is full or not;
+// the workgroup form's time is close to linear in the row pairs.  With the
+// latter in row pairs, a round costs least + PW_IDLE of them and the
+// workgroup form PW_IDLE before its first.  `least` is measured per plan
+// (PW_SMALL and so on); the CFL form spills more and its rounds take a sixth
+// longer.  FP32, workgroup -> wave form: 16 shells of 64 x 128 (512 row
+// pairs) 26 -> 42 us, so workgroup; 96 shells 64 -> 45 us, so wave; at n =
+// 512, 20 shells of 256 points 85 -> 90 us (the second round a quarter full),
+// 32 shells 127 -> 105, 96 shells 353 -> 311 us.
+constexpr long PW_IDLE = 500;
+template <class PL>
+bool physwave_pays(const Ctx& c, long least, bool cfl) {
+    constexpr int by_regs = 4 * PL::WPE / PL::W, by_lds = (int)(163840 / PL::LDS);
+    constexpr int wg = by_regs < 1 || by_lds < 1 ? 1 : by_regs < by_lds ? by_regs : by_lds;
+    const long rows = (long)c.N * c.Th2, round = (long)c.ncu * wg * PL::RP;
+    const long cost = least == 0 ? 0 : (cfl ? least * 6 / 5 : least) + PW_IDLE;
+    return (rows + round - 1) / round * cost <= rows + PW_IDLE;
+}
+
 template <typename R, int N_, int R0_, int R1_, int P_>
-int physwave_run(Ctx& c, PwArgs<R>& a, bool cfl) {
+int physwave_run(Ctx& c, PwArgs<R>& a, bool cfl, long least) {
     typedef PwPlan<(int)sizeof(typename Cx<R>::t), N_, R0_, R1_, P_> PL;
+    if (!physwave_pays<PL>(c, least, cfl)) return 1;
     a.gpr = (c.Th2 + PL::RP - 1) / PL::RP;
     a.nwork = c.N * a.gpr;
     const dim3 g((unsigned)((a.nwork + 7) / 8 * 8));
@@ -641,37 +663,41 @@ int physwave_run(Ctx& c, PwArgs<R>& a, bool cfl) {
     return LSD_OK;
 }
 
-// The lengths each source file instantiates; 1: not one of them.
+// The lengths each source file instantiates; 1: not one of them, or too few
+// row pairs.
 int physwave_f32_small(Ctx& c, PwArgs<float>& a, bool cfl);
 int physwave_f32_large(Ctx& c, PwArgs<float>& a, bool cfl);
 int physwave_f32_long(Ctx& c, PwArgs<float>& a, bool cfl);
 
-#define PW_CASE(R, n, r0, r1, p) \
-    case n: return physwave_run<R, n, r0, r1, p>(c, a, cfl)
+#define PW_CASE(R, n, r0, r1, p, least) \
+    case n: return physwave_run<R, n, r0, r1, p>(c, a, cfl, least)
 
 // Radices: the first at most one butterfly per lane, the last (points per
 // lane) 6 to 9 where the length allows, so that three vectors stay in
-// registers, with as many of the 64 lanes in use as the factors give.
+// registers, with as many of the 64 lanes in use as the factors give.  Last,
+// the row pairs from which a plan beats the workgroup form (0: from one
+// shell's on, measured from 7 shells), at L = M = n / 3 with both vector
+// fields, codensity and composition.
 #define PW_SMALL(R)               \
-    PW_CASE(R, 36, 6, 1, 6);      \
-    PW_CASE(R, 48, 8, 1, 6);      \
-    PW_CASE(R, 54, 9, 1, 6);      \
-    PW_CASE(R, 64, 8, 1, 8);      \
-    PW_CASE(R, 72, 9, 1, 8);      \
-    PW_CASE(R, 96, 12, 1, 8);     \
-    PW_CASE(R, 108, 12, 1, 9);    \
-    PW_CASE(R, 128, 16, 1, 8);    \
-    PW_CASE(R, 144, 16, 1, 9);    \
-    PW_CASE(R, 162, 18, 1, 9);    \
-    PW_CASE(R, 192, 8, 4, 6);     \
-    PW_CASE(R, 216, 9, 3, 8)
+    PW_CASE(R, 36, 6, 1, 6, 650);      \
+    PW_CASE(R, 48, 8, 1, 6, 670);      \
+    PW_CASE(R, 54, 9, 1, 6, 560);      \
+    PW_CASE(R, 64, 8, 1, 8, 2450);      \
+    PW_CASE(R, 72, 9, 1, 8, 720);      \
+    PW_CASE(R, 96, 12, 1, 8, 1100);     \
+    PW_CASE(R, 108, 12, 1, 9, 1200);    \
+    PW_CASE(R, 128, 16, 1, 8, 2000);    \
+    PW_CASE(R, 144, 16, 1, 9, 1200);    \
+    PW_CASE(R, 162, 18, 1, 9, 900);    \
+    PW_CASE(R, 192, 8, 4, 6, 620);     \
+    PW_CASE(R, 216, 9, 3, 8, 660)
 #define PW_LARGE(R)               \
-    PW_CASE(R, 256, 8, 4, 8);     \
-    PW_CASE(R, 288, 8, 6, 6);     \
-    PW_CASE(R, 324, 9, 6, 6);     \
-    PW_CASE(R, 384, 8, 8, 6);     \
-    PW_CASE(R, 432, 9, 6, 8);     \
-    PW_CASE(R, 486, 9, 6, 9);     \
-    PW_CASE(R, 512, 8, 8, 8)
+    PW_CASE(R, 256, 8, 4, 8, 900);     \
+    PW_CASE(R, 288, 8, 6, 6, 0);     \
+    PW_CASE(R, 324, 9, 6, 6, 0);     \
+    PW_CASE(R, 384, 8, 8, 6, 0);     \
+    PW_CASE(R, 432, 9, 6, 8, 0);     \
+    PW_CASE(R, 486, 9, 6, 9, 0);     \
+    PW_CASE(R, 512, 8, 8, 8, 1343)
 
 }  // namespace lsd

@@ -1,6 +1,8 @@
-"""Physical-space pass over phi lengths: the wave form at every length it is
-instantiated for, at the largest M of the 3/2 rule and past it (workgroup
-form), with theta counts that leave row pairs over, against the C oracle.
+"""Physical-space pass over phi lengths against the C oracle: the wave form at
+every length it is instantiated for, at the largest M of the 3/2 rule, with
+theta counts that leave row pairs over, and the workgroup form past the 3/2
+rule, at other lengths and for launches with few row pairs (shells times half
+the theta points), where it is the faster one up to n = 256 and at 512.
 
 The nonlinear terms of one timestep are compared per field, relative to the
 field's norm, at dt = 1e-4 (they are those of the predicted state, whose wall
@@ -14,7 +16,7 @@ import pytest
 
 import oracle_lib
 from lsd import make_config, seeded_state, MIXED_F32, PLAIN_F64
-from lsd.gpu import Context
+from lsd.gpu import Context, K_PHYS
 
 pytestmark = pytest.mark.gpu
 
@@ -55,8 +57,7 @@ def config(Ph, M, precision, Th, **kw):
 @pytest.mark.parametrize("precision,bound", [(PLAIN_F64, 1e-11), (MIXED_F32, 5e-6)])
 def test_lengths(Ph, precision, bound):
     M = Ph // 3 // 2 * 2
-    # 3 and 11 row pairs: one partial workgroup, and whole ones with a rest
-    # or a single partial one, by the row pairs a workgroup takes
+    # 3 and 11 row pairs of 8 shells
     compare(config(Ph, M, precision, 6), bound)
     compare(config(Ph, M - 2, precision, 22, comp=0), bound)
 
@@ -80,3 +81,48 @@ def test_workgroup_form(Ph, M, precision, bound):
 @pytest.mark.parametrize("mag", (0, 1))
 def test_cfl(Ph, precision, bound, mag):
     compare(config(Ph, Ph // 3 // 2 * 2, precision, 14, dt=-1e-6, mag=mag), bound)
+
+
+# row pairs from which the wave form runs (the CFL form from a fifth more; at
+# n = 512 its second round starts at 2048 row pairs); 0: from one shell's on
+LEAST = {36: 650, 48: 670, 54: 560, 64: 2450, 72: 720, 96: 1100, 108: 1200, 128: 2000, 144: 1200, 162: 900,
+         192: 620, 216: 660, 256: 900, 288: 0, 324: 0, 384: 0, 432: 0, 486: 0, 512: 1343}
+
+
+@pytest.mark.parametrize("Ph", SHORT)
+@pytest.mark.parametrize("adapt", (0, 1))
+def test_wave_form(Ph, adapt):
+    """As many shells of 3 and 11 row pairs (one partial workgroup, and whole
+    ones with a rest or a single partial one, by the row pairs that a workgroup
+    takes) as the wave form needs, up to 128, and then more row pairs."""
+    M = Ph // 3 // 2 * 2
+    need = LEAST[Ph] * 6 // 5 + 1
+    for Th2, kw in ((3, {}), (11, {"comp": 0, "mag": 0})):
+        N = min(128, max(8, -(-need // Th2)))
+        Th2 += 2 * max(0, -(-(need - N * Th2) // (2 * N)))
+        assert need <= N * Th2 <= (2048 if Ph == 512 else 1 << 20)
+        compare(config(Ph, M, MIXED_F32, 2 * Th2, N=N, **(dict(kw, dt=-1e-6) if adapt else kw)), 5e-6)
+
+
+@pytest.mark.parametrize("Ph", (36, 64, 108, 128, 162))
+@pytest.mark.parametrize("adapt", (0, 1))
+def test_small_launch_time(Ph, adapt):
+    """On 8 shells the pass of the mixed form takes no longer than that of the
+    plain form, which has the workgroup form only (measured: 0.86 to 0.93 of
+    it; the wave form 1.1 to 1.7 times as long)."""
+    M = Ph // 3 // 2 * 2
+    best = {}
+    for precision in (PLAIN_F64, MIXED_F32):
+        cfg = config(Ph, M, precision, (3 * M // 2 + 3) // 4 * 4, dt=-1e-7 if adapt else 1e-7)
+        g = Context(cfg)
+        g.set_state(seeded_state(cfg, 5, 1e-3))
+        g.step(2)
+        times = []
+        for _ in range(7):
+            g.profile_begin(K_PHYS)
+            g.step(3)
+            ms, launches, _ = g.profile_end()
+            times.append(ms / launches)
+        best[precision] = sorted(times)[3]
+        g.close()
+    assert best[MIXED_F32] <= 1.1 * best[PLAIN_F64], best
