@@ -104,6 +104,17 @@ static bool pageable(const void* p) {
     return a.type == hipMemoryTypeUnregistered;
 }
 
+// Result arrays that share memory: the last part's data are to stay, so the
+// parts go one after another.
+static bool overlap(const HostPart* parts, int np) {
+    for (int k = 0; k < np; k++)
+        for (int q = 0; q < k; q++) {
+            const uintptr_t a = (uintptr_t)parts[k].host, b = (uintptr_t)parts[q].host;
+            if (a < b + parts[q].bytes && b < a + parts[k].bytes) return true;
+        }
+    return false;
+}
+
 // to_host: on return the host arrays hold the data; otherwise the host arrays
 // have been read and the copies are in the stream's order.
 int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host) {
@@ -118,6 +129,7 @@ int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, 
         nq += (parts[k].bytes + HC_CHUNK - 1) / HC_CHUNK;
     }
     for (int k = 0; k < np && total >= HC_MIN; k++) chunks = chunks && pageable(parts[k].host);
+    if (to_host && overlap(parts, np)) chunks = false;
     if (total < HC_MIN || !chunks) {
         for (int k = 0; k < np; k++)
             LSD_HIP(hipMemcpyAsync(to_host ? parts[k].host : parts[k].dev, to_host ? parts[k].dev : parts[k].host,

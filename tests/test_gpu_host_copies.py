@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from lsd import make_config
-from lsd.gpu import Context, Mlp
+from lsd.gpu import Context, Mlp, _p
 
 pytestmark = pytest.mark.gpu
 
@@ -24,6 +24,27 @@ def test_state_fields(L, N):
     for k in (0, 1, 2, 4, 5):
         re, im = g.get_coll(k)
         assert np.array_equal(re, want[k][0]) and np.array_equal(im, want[k][1])
+    g.close()
+
+
+def test_one_array_for_two_results():
+    """A caller that wants one of the results passes its array twice: it gets
+    the later one."""
+    cfg = make_config(L=64, M=64, N=96, dt=1e-6)
+    g = Context(cfg)
+    H = cfg.sizes()[0]
+    re, im = np.random.default_rng(3).standard_normal((2, H, 96))
+    g.set_coll(4, re, im)
+    buf = np.zeros((H, 96))
+    for _ in range(3):
+        assert g.lib.lsd_get_coll(g.h, 4, _p(buf), _p(buf)) == 0
+        assert np.array_equal(buf, im)
+    sre, sim = np.ascontiguousarray(re.T), np.ascontiguousarray(im.T)
+    want = g.grad(sre, sim)[1]
+    p = np.zeros_like(want)
+    for _ in range(3):
+        assert g.lib.lsd_tra_grad(g.h, _p(sre), _p(sim), _p(p), _p(p)) == 0
+        assert np.array_equal(p, want)
     g.close()
 
 
