@@ -5,7 +5,9 @@
 // columns, then one workgroup per output (total, degree, order) sums over the
 // harmonics; the order of every sum is fixed.
 #include <algorithm>
+#include <memory>
 #include <mutex>
+#include <new>
 
 #include "lsd_internal.h"
 
@@ -121,12 +123,16 @@ int energy_run(Ctx& c, int which, double* scratch, double* E, double* El, double
                        c.d_mslot, efac, d_eh, d_out);
     LSD_HIP(hipGetLastError());
     // one copy for the total and both spectra
-    std::vector<double> h_out(nt);
-    LSD_HIP(hipMemcpyAsync(h_out.data(), d_out, sizeof(double) * nt, hipMemcpyDeviceToHost, c.stream));
+    const std::unique_ptr<double[]> h_out(new (std::nothrow) double[nt]);
+    if (!h_out) {
+        set_error("lsd_energy: out of host memory");
+        return LSD_E_HIP;
+    }
+    LSD_HIP(hipMemcpyAsync(h_out.get(), d_out, sizeof(double) * nt, hipMemcpyDeviceToHost, c.stream));
     LSD_HIP(hipStreamSynchronize(c.stream));
     *E = h_out[0];
-    if (El) std::copy(h_out.begin() + 1, h_out.begin() + 1 + c.L, El);
-    if (Em) std::copy(h_out.begin() + 1 + c.L, h_out.end(), Em);
+    if (El) std::copy(&h_out[1], &h_out[1] + c.L, El);
+    if (Em) std::copy(&h_out[1] + c.L, &h_out[1] + c.L + c.M, Em);
     return LSD_OK;
 }
 

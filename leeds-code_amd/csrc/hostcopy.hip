@@ -12,7 +12,7 @@
 // N = 64, 96 x 192 (69 MB): 5.6 -> 3.4 ms; the closure network on 57792 rows
 // of 92 values: 0.98-1.05 -> 0.96 ms, its first call 1.8 -> 1.2 ms.
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 
 #include "lsd_internal.h"
@@ -115,8 +115,10 @@ static bool overlap(const HostPart* parts, int np) {
     return false;
 }
 
-// to_host: on return the host arrays hold the data; otherwise the host arrays
-// have been read and the copies are in the stream's order.
+// to_host: on return the host arrays hold the data.  Otherwise the copies are
+// in the stream's order; they may still read the host arrays (pinned ones, of
+// any size), and on an error copies either way may be under way.  The calling
+// entry point waits for the stream before it returns (CopyGuard).
 int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host) {
     size_t total = 0, nq = 0;
     bool chunks = true;
@@ -147,8 +149,9 @@ int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, 
     for (int t = 1; t < HC_THREADS; t++) {
         try {
             th[t] = std::thread(share, t);
-        } catch (const std::system_error&) {
-            // no thread to be had: the caller's takes the share below
+        } catch (const std::exception&) {
+            // no thread to be had, or no memory for one: the caller's takes
+            // the share below
         }
     }
     share(0);

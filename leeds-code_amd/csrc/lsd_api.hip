@@ -1307,10 +1307,11 @@ int lsd_set_coll(lsd_ctx* ctx, int field, const double* re, const double* im) {
     }
     const size_t HN = c.coll_elems();
     double* tmp = lsd::coll_staging(c);
+    lsd::CopyGuard guard(c.stream);
     int rc = lsd::copy_pair(c, re, im, tmp, false);
     if (rc || (rc = lsd::launch_merge_coll(c, tmp, tmp + HN, c.d_f[field]))) return rc;
     LSD_HIP(hipStreamSynchronize(c.stream));
-    return LSD_OK;
+    return guard.pass(LSD_OK);
 }
 
 int lsd_set_ic(lsd_ctx* ctx, int which, const double* re, const double* im) {
@@ -1511,8 +1512,9 @@ int lsd_get_coll(lsd_ctx* ctx, int field, double* re, double* im) {
     }
     const size_t HN = c.coll_elems();
     double* tmp = lsd::coll_staging(c);
+    lsd::CopyGuard guard(c.stream);
     int rc = lsd::launch_split_coll(c, c.d_f[field], tmp, tmp + HN);
-    return rc ? rc : lsd::copy_pair(c, re, im, tmp, true);
+    return rc ? rc : guard.pass(lsd::copy_pair(c, re, im, tmp, true));
 }
 
 int lsd_get_phys(lsd_ctx* ctx, int field, double* p) {
@@ -1522,7 +1524,8 @@ int lsd_get_phys(lsd_ctx* ctx, int field, double* p) {
         return LSD_E_ARG;
     }
     const lsd::HostPart part = {p, lsd::phys(c, field), sizeof(double) * c.phys_elems()};
-    return lsd::host_copy(c.stage, c.stream, &part, 1, true);
+    lsd::CopyGuard guard(c.stream);
+    return guard.pass(lsd::host_copy(c.stage, c.stream, &part, 1, true));
 }
 
 int lsd_get_table(lsd_ctx* ctx, int table, double* out) {
@@ -1825,16 +1828,18 @@ int lsd_sht_roundtrip(lsd_ctx* ctx, int kind, const double* in, double* out) {
 
 int lsd_tra_spec2phys(lsd_ctx* ctx, const double* s_re, const double* s_im, double* p) {
     CTX_OR_FAIL(ctx);
+    lsd::CopyGuard guard(c.stream);
     int rc;
     double2* in = lsd::spec_in(c, lsd::SI_DC);
     if ((rc = lsd::upload_spec(c, 1, &s_re, &s_im, &in))) return rc;
     if ((rc = lsd::launch_synthesis(c, lsd::SYN_SCALAR, in, nullptr, lsd::fourier(c, 0), nullptr))) return rc;
     if ((rc = lsd::launch_fft_c2r(c, lsd::fourier(c, 0), lsd::phys(c, 0), 1))) return rc;
-    return lsd::copy_phys(c, 1, &p, true);
+    return guard.pass(lsd::copy_phys(c, 1, &p, true));
 }
 
 int lsd_tra_grad(lsd_ctx* ctx, const double* s_re, const double* s_im, double* t, double* p) {
     CTX_OR_FAIL(ctx);
+    lsd::CopyGuard guard(c.stream);
     int rc;
     double2* in = lsd::spec_in(c, lsd::SI_DC);
     if ((rc = lsd::upload_spec(c, 1, &s_re, &s_im, &in))) return rc;
@@ -1842,12 +1847,13 @@ int lsd_tra_grad(lsd_ctx* ctx, const double* s_re, const double* s_im, double* t
         return rc;
     if ((rc = lsd::launch_fft_c2r(c, lsd::fourier(c, 0), lsd::phys(c, 0), 2))) return rc;
     const double* out[2] = {t, p};
-    return lsd::copy_phys(c, 2, out, true);
+    return guard.pass(lsd::copy_phys(c, 2, out, true));
 }
 
 int lsd_tra_qst2rtp(lsd_ctx* ctx, const double* q_re, const double* q_im, const double* s_re, const double* s_im,
                     const double* t_re, const double* t_im, double* r, double* th, double* ph) {
     CTX_OR_FAIL(ctx);
+    lsd::CopyGuard guard(c.stream);
     int rc;
     double2* q = lsd::spec_in(c, lsd::SI_UQ);
     double2* s = lsd::spec_in(c, lsd::SI_US);
@@ -1860,11 +1866,12 @@ int lsd_tra_qst2rtp(lsd_ctx* ctx, const double* q_re, const double* q_im, const 
     if ((rc = lsd::launch_synthesis(c, lsd::SYN_VECTOR, s, t, lsd::fourier(c, 1), lsd::fourier(c, 2)))) return rc;
     if ((rc = lsd::launch_fft_c2r(c, lsd::fourier(c, 0), lsd::phys(c, 0), 3))) return rc;
     const double* out[3] = {r, th, ph};
-    return lsd::copy_phys(c, 3, out, true);
+    return guard.pass(lsd::copy_phys(c, 3, out, true));
 }
 
 int lsd_tra_phys2spec(lsd_ctx* ctx, const double* p, double* s_re, double* s_im) {
     CTX_OR_FAIL(ctx);
+    lsd::CopyGuard guard(c.stream);
     int rc;
     double* x = lsd::phys(c, 0);
     if ((rc = lsd::copy_phys(c, 1, &p, false))) return rc;
@@ -1872,12 +1879,13 @@ int lsd_tra_phys2spec(lsd_ctx* ctx, const double* p, double* s_re, double* s_im)
     double2* o = lsd::spec_out(c, lsd::SO_C);
     if ((rc = lsd::launch_analysis(c, lsd::ANA_SCALAR, lsd::folded(c, 0), nullptr, nullptr, o, nullptr, nullptr)))
         return rc;
-    return lsd::download_spec(c, 1, &o, &s_re, &s_im);
+    return guard.pass(lsd::download_spec(c, 1, &o, &s_re, &s_im));
 }
 
 int lsd_tra_rtp2qst(lsd_ctx* ctx, const double* r, const double* th, const double* ph, double* q_re, double* q_im,
                     double* s_re, double* s_im, double* t_re, double* t_im) {
     CTX_OR_FAIL(ctx);
+    lsd::CopyGuard guard(c.stream);
     int rc;
     const double* in[3] = {r, th, ph};
     if ((rc = lsd::copy_phys(c, 3, in, false))) return rc;
@@ -1891,7 +1899,7 @@ int lsd_tra_rtp2qst(lsd_ctx* ctx, const double* r, const double* th, const doubl
     const double2* o[3] = {o0, o1, o2};
     double* re[3] = {q_re, s_re, t_re};
     double* im[3] = {q_im, s_im, t_im};
-    return lsd::download_spec(c, 3, o, re, im);
+    return guard.pass(lsd::download_spec(c, 3, o, re, im));
 }
 
 }  // extern "C"

@@ -60,6 +60,23 @@ struct HostPart {
 };
 int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host);
 
+// Waits for the stream on every return of a call with host arrays but a
+// successful one (which waits itself): no copy still reads or writes the
+// caller's arrays when the call has returned.
+struct CopyGuard {
+    hipStream_t stream;
+    bool passed = false;
+    explicit CopyGuard(hipStream_t s) : stream(s) {}
+    CopyGuard(const CopyGuard&) = delete;
+    ~CopyGuard() {
+        if (!passed) (void)hipStreamSynchronize(stream);
+    }
+    int pass(int rc) {
+        passed = rc == LSD_OK;
+        return rc;
+    }
+};
+
 // Stream-ordered scratch of a set-up or diagnostic call, returned to the
 // pool on every exit path (the call synchronises the stream before using
 // what the kernels wrote, so the free follows all uses).

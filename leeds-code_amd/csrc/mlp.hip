@@ -937,15 +937,17 @@ int lsd_mlp_forward(lsd_mlp* m, long rows, const float* x, float* y) {
     if (rc) return rc;
     const lsd::HostPart in = {const_cast<float*>(x), m->X, sizeof(float) * rows * m->nin};
     const lsd::HostPart out = {y, m->Y, sizeof(float) * rows * m->nout};
+    lsd::CopyGuard guard(m->stream);
     if ((rc = lsd::host_copy(m->stage, m->stream, &in, 1, false))) return rc;
     if ((rc = mlp_forward_dev(m, rows, m->X, false))) return rc;
-    return lsd::host_copy(m->stage, m->stream, &out, 1, true);
+    return guard.pass(lsd::host_copy(m->stage, m->stream, &out, 1, true));
 }
 
 int lsd_mlp_grad(lsd_mlp* m, long rows, const float* x, const float* target, float* loss, float* grad) {
     if (!m || !x || !target || rows < 1) { lsd::set_error("lsd_mlp_grad: bad arguments"); return LSD_E_ARG; }
     int rc = mlp_rows(m, rows);
     if (rc) return rc;
+    lsd::CopyGuard guard(m->stream);
     LSD_HIP(hipMemcpyAsync(m->X, x, sizeof(float) * rows * m->nin, hipMemcpyHostToDevice, m->stream));
     LSD_HIP(hipMemcpyAsync(m->T, target, sizeof(float) * rows * m->nout, hipMemcpyHostToDevice, m->stream));
     if ((rc = mlp_forward_dev(m, rows, m->X, true))) return rc;
@@ -953,7 +955,7 @@ int lsd_mlp_grad(lsd_mlp* m, long rows, const float* x, const float* target, flo
     if (loss && (rc = mlp_losses(m, 1, &rows, loss))) return rc;
     if (grad) LSD_HIP(hipMemcpyAsync(grad, m->g, sizeof(float) * m->np, hipMemcpyDeviceToHost, m->stream));
     LSD_HIP(hipStreamSynchronize(m->stream));
-    return LSD_OK;
+    return guard.pass(LSD_OK);
 }
 
 // Adam steps on minibatches drawn in order from (x, target) [rows x n],
@@ -975,6 +977,7 @@ int lsd_mlp_train(lsd_mlp* m, long rows, const float* x, const float* target, lo
     }
     int rc = mlp_rows(m, batch);
     if (rc) return rc;
+    lsd::CopyGuard guard(m->stream);
     LSD_HIP(hipMemcpyAsync(m->sx, x, sizeof(float) * rows * m->nin, hipMemcpyHostToDevice, m->stream));
     LSD_HIP(hipMemcpyAsync(m->st, target, sizeof(float) * rows * m->nout, hipMemcpyHostToDevice, m->stream));
     long pos = 0;
@@ -1000,7 +1003,7 @@ int lsd_mlp_train(lsd_mlp* m, long rows, const float* x, const float* target, lo
         }
     }
     LSD_HIP(hipStreamSynchronize(m->stream));
-    return rc;
+    return guard.pass(rc);
 }
 
 }  // extern "C"

@@ -26,8 +26,13 @@ std::mutex mu;
 std::deque<Op> queue;
 std::map<const char*, size_t> pinned;
 std::thread::id caller;
+thread_local bool in_runtime = false;
+struct Lock {
+    std::lock_guard<std::mutex> g{mu};
+    Lock() { in_runtime = true; }
+    ~Lock() { in_runtime = false; }
+};
 int caller_delay_ms = 0, copies_ok = -1, threads_fail = 0;
-thread_local bool in_thread_start = false;
 
 bool is_pinned(const void* p) {
     auto it = pinned.upper_bound((const char*)p);
@@ -49,7 +54,7 @@ void run_until(hipEvent_t ev) {
 
 extern "C" {
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind kind, hipStream_t) {
-    std::lock_guard<std::mutex> g(mu);
+    Lock lock;
     if (copies_ok == 0) return hipErrorInvalidValue;
     if (copies_ok > 0) copies_ok--;
     queue.push_back({dst, src, n, nullptr});
@@ -57,7 +62,7 @@ hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind ki
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t) {
-    std::lock_guard<std::mutex> g(mu);
+    Lock lock;
     run_until(nullptr);
     return hipSuccess;
 }
@@ -70,7 +75,7 @@ hipError_t hipEventDestroy(hipEvent_t e) {
     return hipSuccess;
 }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
-    std::lock_guard<std::mutex> g(mu);
+    Lock lock;
     for (Op& o : queue)
         if (o.ev == e) o.ev = nullptr;
     queue.push_back({nullptr, nullptr, 0, e});
@@ -79,18 +84,18 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
 hipError_t hipEventSynchronize(hipEvent_t e) {
     if (caller_delay_ms && std::this_thread::get_id() == caller)
         std::this_thread::sleep_for(std::chrono::milliseconds(caller_delay_ms));
-    std::lock_guard<std::mutex> g(mu);
+    Lock lock;
     run_until(e);
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     *p = malloc(n);
-    std::lock_guard<std::mutex> g(mu);
+    Lock lock;
     pinned[(const char*)*p] = n;
     return hipSuccess;
 }
 hipError_t hipHostFree(void* p) {
-    std::lock_guard<std::mutex> g(mu);
+    Lock lock;
     run_until(nullptr);  // as the runtime waits for the device
     pinned.erase((const char*)p);
     free(p);
@@ -98,7 +103,7 @@ hipError_t hipHostFree(void* p) {
 }
 #undef hipPointerGetAttributes
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
-    std::lock_guard<std::mutex> g(mu);
+    Lock lock;
     memset(a, 0, sizeof *a);
     a->type = is_pinned(p) ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
     return hipSuccess;
@@ -112,9 +117,9 @@ hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
 }
 
-// a thread's state is allocated before the thread starts
+// a thread's state is allocated by the thread that starts it
 void* operator new(size_t n) {
-    if (threads_fail && std::this_thread::get_id() == caller && in_thread_start) throw std::bad_alloc();
+    if (threads_fail && !in_runtime && std::this_thread::get_id() == caller) throw std::bad_alloc();
     if (void* p = malloc(n)) return p;
     throw std::bad_alloc();
 }
@@ -141,9 +146,12 @@ int fake_host_copy(int np, void** host, void** dev, const size_t* bytes, int to_
         if (pin) pinned[(const char*)host[k]] = bytes[k];
     }
     threads_fail = oom;
-    in_thread_start = oom != 0;
-    const int rc = lsd::host_copy(st, nullptr, parts, np, to_host != 0);
-    in_thread_start = false;
+    int rc;
+    try {
+        rc = lsd::host_copy(st, nullptr, parts, np, to_host != 0);
+    } catch (const std::exception&) {
+        rc = -99;  // through a C entry point this would end the program
+    }
     threads_fail = 0;
     copies_ok = -1;
     caller_delay_ms = 0;

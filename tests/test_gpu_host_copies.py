@@ -2,8 +2,11 @@
 they go through pinned chunks, with a last chunk of one element, whole chunks
 and a rest: state fields set and read back, exactly; both directions of the
 network's forward pass against slices small enough for the plain copy."""
+import time
+
 import numpy as np
 import pytest
+import torch
 
 from lsd import make_config
 from lsd.gpu import Context, Mlp, _p
@@ -55,3 +58,20 @@ def test_network_forward(rows):
     y = net.forward(x)
     for r in range(0, rows, 5000):
         assert np.array_equal(y[r:r + 5000], net.forward(x[r:r + 5000]))
+
+
+def test_failed_call_has_read_its_pinned_array():
+    """A call that fails after its upload was queued returns when the upload is
+    done: 190 MB of pinned memory, which may be read until the stream is waited
+    for, take more than 190 MB / 100 GB/s on the link."""
+    cfg = make_config(L=260, M=2, N=128, Th=390, Ph=486, dt=1e-6)
+    g = Context(cfg)
+    p = torch.ones((128, 486, 390), dtype=torch.float64, pin_memory=True).numpy()
+    out = np.zeros((2, 128, cfg.sizes()[0]))
+    for _ in range(2):
+        t = time.perf_counter()
+        rc = g.lib.lsd_tra_phys2spec(g.h, _p(p), _p(out[0]), _p(out[1]))
+        t = time.perf_counter() - t
+        assert rc != 0 and b"too large" in g.lib.lsd_last_error()
+        assert t >= p.nbytes / 100e9
+    g.close()

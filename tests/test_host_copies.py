@@ -65,3 +65,14 @@ def test_overlapping_results(lib, offset, delay):
     buf = np.zeros(n + offset, dtype=np.uint8)
     assert copy(lib, [buf[:n], buf[offset:]], dev, True, delay=delay) == 0
     assert np.all(buf[offset:] == 2) and np.all(buf[:offset] == 1)
+
+
+@pytest.mark.parametrize("to_host", [True, False])
+def test_no_memory_for_threads(lib, to_host):
+    """Without memory for a thread's state the calling thread does the work: no
+    exception leaves the copy."""
+    src = np.random.default_rng(2).integers(0, 256, 7 * MB + 1, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    host, dev = (dst, src) if to_host else (src, dst)
+    assert copy(lib, [host], [dev], to_host, oom=True) == 0
+    assert np.array_equal(src, dst)
