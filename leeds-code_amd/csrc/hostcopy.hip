@@ -21,8 +21,13 @@ namespace lsd {
 
 constexpr int HC_THREADS = 4;  // eight gain nothing: mapping the pages takes turns
 constexpr size_t HC_CHUNK = size_t(1) << 20;
-// below this the threads' start (about 50 us) costs more than they save
-constexpr size_t HC_MIN = size_t(2) << 20;
+// From these sizes on the threads' start (about 50 us) is made up for, also for
+// arrays that the caller keeps from call to call.  Results, 2.4 MB: 212 us
+// directly, 189 through the chunks; new arrays 606 and 433.  Uploads find
+// their pages mapped and gain later, analysis of one field and of three: 4.7 MB
+// 253 us directly, 346 through the chunks; 18.9 MB 770 and 883 (new arrays
+// 940, 920), 28.3 MB 1140-1380 and 1302 (1410, 1340), 56.6 MB 2595 and 2448.
+constexpr size_t HC_MIN = size_t(2) << 20, HC_MIN_UP = size_t(24) << 20;
 
 int HostStage::reserve() {
     if (buf) return LSD_OK;
@@ -121,7 +126,6 @@ static bool overlap(const HostPart* parts, int np) {
 // entry point waits for the stream before it returns (CopyGuard).
 int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host) {
     size_t total = 0, nq = 0;
-    bool chunks = true;
     for (int k = 0; k < np; k++) {
         if (!parts[k].host) {
             set_error("null host array");
@@ -130,9 +134,10 @@ int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, 
         total += parts[k].bytes;
         nq += (parts[k].bytes + HC_CHUNK - 1) / HC_CHUNK;
     }
-    for (int k = 0; k < np && total >= HC_MIN; k++) chunks = chunks && pageable(parts[k].host);
+    bool chunks = total >= (to_host ? HC_MIN : HC_MIN_UP);
+    for (int k = 0; k < np && chunks; k++) chunks = pageable(parts[k].host);
     if (to_host && overlap(parts, np)) chunks = false;
-    if (total < HC_MIN || !chunks) {
+    if (!chunks) {
         for (int k = 0; k < np; k++)
             LSD_HIP(hipMemcpyAsync(to_host ? parts[k].host : parts[k].dev, to_host ? parts[k].dev : parts[k].host,
                                    parts[k].bytes, to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, stream));

@@ -14,8 +14,10 @@ from lsd.gpu import Context, Mlp, _p
 pytestmark = pytest.mark.gpu
 
 
-# H = 528 (L = 32) and 4656 (L = 96) coll rows: 2 x 8 x H N bytes a field
-@pytest.mark.parametrize("L,N", [(32, 7), (32, 31), (32, 248), (32, 249), (32, 256), (96, 127)])
+# H = 528 (L = 32) and 4656 (L = 96) coll rows: 2 x 8 x H N bytes a field, from
+# 59 KB to 25 MB
+@pytest.mark.parametrize("L,N", [(32, 7), (32, 31), (32, 248), (32, 249), (32, 256), (96, 10),
+                                 (96, 11), (96, 127), (96, 339)])
 def test_state_fields(L, N):
     cfg = make_config(L=L, M=L, N=N, dt=1e-6)
     g = Context(cfg)
@@ -51,7 +53,21 @@ def test_one_array_for_two_results():
     g.close()
 
 
-@pytest.mark.parametrize("rows", [1000, 32768, 32769, 70001])
+def test_transform_uploads():
+    """rtp -> qst and back of 28 MB of pageable arrays, in chunks, and of pinned
+    ones, directly: the same bits."""
+    cfg = make_config(L=64, M=64, N=65, dt=1e-6)
+    g = Context(cfg)
+    p = [torch.randn((65, g.Ph, g.Th), dtype=torch.float64, generator=torch.Generator().manual_seed(k)) for k in range(3)]
+    assert 3 * p[0].numel() * 8 > 24 << 20
+    a = g.rtp2qst(*[x.numpy() for x in p])
+    b = g.rtp2qst(*[x.pin_memory().numpy() for x in p])
+    for x, y in zip(a, b):
+        assert np.array_equal(x[0], y[0]) and np.array_equal(x[1], y[1])
+    g.close()
+
+
+@pytest.mark.parametrize("rows", [1000, 32768, 32769, 70001, 400001])
 def test_network_forward(rows):
     net = Mlp(16, 32, 16)
     x = np.random.default_rng(rows).standard_normal((rows, 16)).astype(np.float32)

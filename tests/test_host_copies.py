@@ -34,10 +34,10 @@ def copy(lib, host, dev, to_host, pin=False, delay=0, ok=-1, oom=False):
                               S(*[a.nbytes for a in host]), int(to_host), int(pin), delay, ok, int(oom))
 
 
-# below and above the size of the chunked copies, last chunks of 1 byte and of
-# all but one, several parts
+# below and above the sizes of the chunked copies (2 MiB of results, 24 MiB of
+# uploads), last chunks of 1 byte and of all but one, several parts
 SIZES = [(1,), (2 * MB - 1,), (2 * MB,), (5 * MB + 1,), (9 * MB - 1,), (MB, 3 * MB, 1), (4 * MB + 5, 7, 6 * MB),
-         (40 * MB + 3,)]
+         (24 * MB - 1,), (24 * MB + 1,), (12 * MB + 5, 7, 13 * MB - 1)]
 
 
 @pytest.mark.parametrize("sizes", SIZES)
@@ -71,7 +71,7 @@ def test_overlapping_results(lib, offset, delay):
 def test_no_memory_for_threads(lib, to_host):
     """Without memory for a thread's state the calling thread does the work: no
     exception leaves the copy."""
-    src = np.random.default_rng(2).integers(0, 256, 7 * MB + 1, dtype=np.uint8)
+    src = np.random.default_rng(2).integers(0, 256, 25 * MB + 1, dtype=np.uint8)
     dst = np.zeros_like(src)
     host, dev = (dst, src) if to_host else (src, dst)
     assert copy(lib, [host], [dev], to_host, oom=True) == 0
