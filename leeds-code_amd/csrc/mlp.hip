@@ -571,6 +571,7 @@ struct lsd_mlp {
     float *dY = nullptr, *dZ1 = nullptr, *dZ2 = nullptr, *part = nullptr;
     float *sx = nullptr, *st = nullptr;
     float* h_part = nullptr;
+    int slots = 0;  // steps whose loss partials fit part and h_part
     // packed weights of the fused passes
     __bf16* pk = nullptr;
     bool fused() const { return nin <= FUSE_MAX && width <= FUSE_MAX && nto() <= mf_tiles(width); }
@@ -599,8 +600,11 @@ struct lsd_mlp {
     long o_b3() const { return o_w3() + (long)nout * width; }
 };
 
-// losses kept on the device before they are copied to the host together
+// Losses of so many steps stay on the device before they are copied to the
+// host together: 256, or as many as LOSS_BYTES hold partials of (one at least).
 constexpr int LOSS_STEPS = 256;
+constexpr long LOSS_BYTES = 4L << 20;
+static int loss_slots(long nb) { return (int)std::max(1L, std::min((long)LOSS_STEPS, LOSS_BYTES / (long)sizeof(float) / nb)); }
 
 static void mlp_free_rows(lsd_mlp* m) {
     float** bufs[] = {&m->Z1, &m->H1, &m->Z2, &m->H2, &m->T, &m->dY, &m->dZ1, &m->dZ2, &m->part};
@@ -647,8 +651,9 @@ static int mlp_rows(lsd_mlp* m, long rows) {
     for (float** b : hid) LSD_HIP(hipMalloc((void**)b, sizeof(float) * rows * W));
     LSD_HIP(hipMalloc((void**)&m->T, sizeof(float) * rows * m->nout));
     LSD_HIP(hipMalloc((void**)&m->dY, sizeof(float) * rows * m->ldy()));
-    LSD_HIP(hipMalloc((void**)&m->part, sizeof(float) * nb * LOSS_STEPS));
-    LSD_HIP(hipHostMalloc((void**)&m->h_part, sizeof(float) * nb * LOSS_STEPS, hipHostMallocDefault));
+    m->slots = loss_slots(nb);
+    LSD_HIP(hipMalloc((void**)&m->part, sizeof(float) * nb * m->slots));
+    LSD_HIP(hipHostMalloc((void**)&m->h_part, sizeof(float) * nb * m->slots, hipHostMallocDefault));
     m->cap = rows;
     return LSD_OK;
 }
@@ -997,7 +1002,7 @@ int lsd_mlp_train(lsd_mlp* m, long rows, const float* x, const float* target, lo
         LSD_HIP(hipGetLastError());
         if (!loss) continue;
         nrows[nl++] = nrow;
-        if (nl == LOSS_STEPS || s + 1 == steps) {
+        if (nl == m->slots || s + 1 == steps) {
             if ((rc = mlp_losses(m, nl, nrows, loss + s + 1 - nl))) break;
             nl = 0;
         }

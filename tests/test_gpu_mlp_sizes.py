@@ -9,6 +9,7 @@ import sys
 
 import numpy as np
 import pytest
+import torch
 
 from lsd.gpu import Mlp
 
@@ -58,4 +59,27 @@ def test_infinite_inputs(width):
     rest = np.ones(40, dtype=bool)
     rest[[5, 39]] = False
     assert np.array_equal(y[rest], want[rest])
+    m.close()
+
+
+def test_memory_and_losses_of_large_batches():
+    """The loss partials add little to the activations (X, Y, T and dY, six
+    arrays of the width; 100000 floats of partials a step here, for which 256
+    steps would take 102 MB), and the losses are right when they are fetched
+    every few steps: with no learning rate those of the two batches in turn."""
+    m = Mlp(4, 4, 64, seed=5)
+    rows = 400000
+    rng = np.random.default_rng(6)
+    X = rng.standard_normal((rows, 4)).astype(np.float32)
+    T = rng.standard_normal((rows, 64)).astype(np.float32)
+    m.forward(X[:8])
+    free = torch.cuda.mem_get_info()[0]
+    m.grad(X, T)
+    used = free - torch.cuda.mem_get_info()[0]
+    assert used <= 4 * rows * (4 + 3 * 64 + 6 * 4) + (32 << 20)
+    half = [m.grad(X[:rows // 2], T[:rows // 2])[0], m.grad(X[rows // 2:], T[rows // 2:])[0]]
+    m.close()
+    m = Mlp(4, 4, 64, seed=5)
+    losses = m.train(X, T, rows // 2, 45, 0.0)
+    assert np.array_equal(losses, np.array((half * 23)[:45], dtype=np.float32))
     m.close()
