@@ -132,12 +132,24 @@ __global__ void k_gelu_back(long n, const float* __restrict__ Z, float* __restri
     if (i < n) d[i] = d[i] * gelu_grad(Z[i]);
 }
 
-// Column sums of dY [rows][ld], cols of each row, into db (bias gradients).
+// Column sums of dY [rows][ld], cols of each row, into db (bias gradients), row
+// by row.  COLSUM_AHEAD rows are loaded before they are added: with one load at
+// a time the sum is a chain of memory latencies, which moved by up to 14 % with
+// the rows' stride and place.
+constexpr int COLSUM_AHEAD = 8;
 __global__ void k_colsum(int rows, int cols, int ld, const float* __restrict__ dY, float* __restrict__ db) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= cols) return;
     float s = 0.f;
-    for (int i = 0; i < rows; i++) s += dY[(long)i * ld + j];
+    int i = 0;
+    for (; i + COLSUM_AHEAD <= rows; i += COLSUM_AHEAD) {
+        float v[COLSUM_AHEAD];
+#pragma unroll
+        for (int e = 0; e < COLSUM_AHEAD; e++) v[e] = dY[(long)(i + e) * ld + j];
+#pragma unroll
+        for (int e = 0; e < COLSUM_AHEAD; e++) s += v[e];
+    }
+    for (; i < rows; i++) s += dY[(long)i * ld + j];
     db[j] = s;
 }
 

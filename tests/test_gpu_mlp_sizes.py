@@ -21,7 +21,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n_in,width,n_out,rows", [
     (92, 256, 10, 1), (92, 256, 10, 33), (92, 256, 10, 513), (92, 250, 10, 129), (17, 48, 3, 640), (93, 200, 33, 127),
-    (92, 128, 10, 1025), (256, 256, 256, 96), (92, 64, 64, 31), (1, 16, 1, 512), (300, 256, 10, 200), (92, 260, 10, 65)])
+    (92, 128, 10, 1025), (256, 256, 256, 96), (92, 64, 64, 31), (1, 16, 1, 512), (300, 256, 10, 200), (92, 260, 10, 65),
+    (300, 20, 3, 7), (300, 20, 3, 8), (92, 64, 65, 1025)])
 def test_sizes(n_in, width, n_out, rows):
     rng = np.random.default_rng(rows + width)
     m = Mlp(n_in, width, n_out, seed=3)
