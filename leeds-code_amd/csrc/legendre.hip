@@ -944,7 +944,7 @@ template <typename T>
 struct AnaArgs {
     int N, Th2, M, H;
     int ncc, ngroups;  // column chunks per job, slots
-    int njob, maxhb;       // jobs, harmonic blocks of the longest class (k_ana8)
+    int njob, tp, maxhb;   // jobs; tiles per wave at most, harmonic blocks of the longest class (k_ana8)
     const Slot* slots;
     const int* order;
     const T* tP;   // gwP        [Th2][H] (parity-grouped h)
@@ -1157,8 +1157,8 @@ k_ana(AnaArgs<T> a) {
 //   products run.
 // The two waves of a workgroup take the two classes of the same shells, which
 // read the same folded rows.
-// Bound: three tiles and 30 MFMAs (1920 cycles) a step against 9.5 KB of
-// operands, from L2 mostly; the barriers and single wave per SIMD of the
+// Bound, in large launches: three tiles and 30 MFMAs (1920 cycles) a step
+// against 9.5 KB of operands, from L2 mostly; the barriers and single wave per SIMD of the
 // LDS-staged form left the matrix cores idle 4 cycles in 5.  L = M = 170,
 // N = 96, both vector fields: 483 -> 264 us (27 of 73 TFLOP/s), scalars 75 ->
 // 70 us; L = M = 32, N = 32: 14.6 -> 6.6 us.
@@ -1285,9 +1285,9 @@ __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2))) k
     const int job = bid.cc / (a.maxhb * a.ncc), rest = bid.cc - job * a.maxhb * a.ncc;
     const int hb = rest / a.ncc, sb = rest - hb * a.ncc;
     const int par = uniform(threadIdx.x >> 6);
-    // the class's tiles in equal shares of at most A8_TP
+    // the class's tiles in equal shares of at most tp
     const int ncls = par ? s.len / 2 : (s.len + 1) / 2;
-    const int tiles = (ncls + 15) / 16, nb = (tiles + A8_TP - 1) / A8_TP;
+    const int tiles = (ncls + 15) / 16, nb = (tiles + a.tp - 1) / a.tp;
     if (hb >= nb) return;
     const int t0 = tiles * hb / nb, nt = tiles * (hb + 1) / nb - t0;
     if (nt == 3) ana8_item<VEC, 3>(a, s, job, sb, par, t0);
@@ -1539,6 +1539,20 @@ static int ana4_launch(Ctx& c, int kind, int njob, const void* const* g0, const 
     return LSD_OK;
 }
 
+// Tiles per wave of k_ana8.  Three read the least; fewer give the CUs more
+// workgroups (two waves each), which pays while they are idle: a launch of few
+// takes as long as its longest wave.  One tile below four workgroups a CU that
+// way, two below five; over L = 32 to 250, N = 7 to 96 no launch is then slower
+// than the LDS-staged form, which three tiles were by up to 25 % at L = 98 to
+// 128.  Vector and scalar analyses of a step (two evaluations), one / two /
+// three tiles, us: L = 100, M = 50, one vector field, N = 16 50 / 65 / 91, N =
+// 64 89 / 94 / 127; L = M = 128, both, N = 20 171 / 146 / 169, N = 96 442 / 355
+// / 365; L = M = 86, both, N = 64 163 / 152 / 134.
+static int ana8_tiles(int tiles, long shares, int ncu) {
+    if (shares * tiles < 4L * ncu) return 1;
+    return shares * ((tiles + 1) / 2) < 5L * ncu ? 2 : A8_TP;
+}
+
 template <typename T>
 static int ana_launch(Ctx& c, int kind, int njob, const T* tP, const T* tL, const T* tS, const void* const* g0,
                       const void* const* g1, const void* const* g2, void* const* o0, void* const* o1,
@@ -1576,7 +1590,9 @@ static int ana_launch(Ctx& c, int kind, int njob, const T* tP, const T* tL, cons
     a.ncc = (2 * c.N + ANA_COLS - 1) / ANA_COLS;
     a.ngroups = c.nslot;
     a.njob = njob;
-    a.maxhb = (((maxlen + 1) / 2 + 15) / 16 + A8_TP - 1) / A8_TP;
+    const int mt = ((maxlen + 1) / 2 + 15) / 16;  // tiles of the longest class
+    a.tp = std::is_same<T, double>::value ? ana8_tiles(mt, (long)a.ngroups * a.ncc * njob, c.ncu) : A8_TP;
+    a.maxhb = (mt + a.tp - 1) / a.tp;
     if constexpr (std::is_same<T, double>::value) {
         static_assert(2 * A8_SH == ANA_COLS, "one shell block per column chunk");
         const dim3 grid(grid_blocks(a.ngroups, a.ncc * a.maxhb * njob));
