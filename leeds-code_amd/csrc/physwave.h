@@ -17,10 +17,10 @@
 // The zero band of the input is never loaded nor multiplied and the outputs
 // beyond M are never formed (3 M <= n, the 3/2 rule).
 //
-// What bounds it: VALU issue (46 % busy at n = 512) and the latency of loads
-// and LDS exchanges at two waves per SIMD, which the three vectors held per
-// lane allow: without its loads the launch at n = 512 takes 244 us, without
-// its stores 284 us, of 313 us.  The workgroup form of this pass
+// What bounds it: VALU issue and the latency of loads and LDS exchanges at two
+// waves per SIMD, which the three vectors held per lane allow: without its
+// loads the launch at n = 512 takes 244 us, without its stores 284 us, of 313
+// us.  The workgroup form of this pass
 // (physfuse.hip: a row pair per workgroup, six fields per batch, a barrier
 // pair per stage) spends its time on index arithmetic, LDS bank conflicts and
 // threads without a point.  FP32, per launch, workgroup -> wave form (L = M,
@@ -167,8 +167,9 @@ struct PwPlan {
     static constexpr int L0 = (R0 + 2) / 3;
     static constexpr int W = G == 1 && BYTES == 8 && P <= 8 ? 8 : 4;  // waves per workgroup
     static constexpr int RP = W * G;                              // row pairs per workgroup
-    // three sets of 3 P complex values stay live: FP32 fits them in half of
-    // the register file up to P = 9
+    // three sets of 3 P complex values stay live, 108 registers at P = 6: two
+    // waves a SIMD up to P = 9, where 162 of 256 registers leave the transforms
+    // too few and some spill (see the plans)
     static constexpr int WPE = BYTES == 8 && P <= 9 ? 2 : 1;
 
     static constexpr int LANES = 256 / BYTES;  // lanes served at once, = element slots over the 64 banks
@@ -624,17 +625,20 @@ __global__ void __launch_bounds__(64 * PL::W) __attribute__((amdgpu_waves_per_eu
     }
 }
 
-// Whether the wave form is the faster one for this launch.  Its time is one
-// row pair's chain of stages per round, a round being the row pairs that the
-// registers and the LDS of all CUs hold, whether the round is full or not;
-// the workgroup form's time is close to linear in the row pairs.  With the
-// latter in row pairs, a round costs least + PW_IDLE of them and the
-// workgroup form PW_IDLE before its first.  `least` is measured per plan
-// (PW_SMALL and so on); the CFL form spills more and its rounds take a sixth
-// longer.  FP32, workgroup -> wave form: 16 shells of 64 x 128 (512 row
-// pairs) 26 -> 42 us, so workgroup; 96 shells 64 -> 45 us, so wave; at n =
-// 512, 20 shells of 256 points 85 -> 90 us (the second round a quarter full),
-// 32 shells 127 -> 105, 96 shells 353 -> 311 us.
+// Whether a launch takes the wave form.  Its time is one row pair's chain of
+// stages per round, a round being the row pairs that the registers and the LDS
+// of all CUs hold, whether the round is full or not; the workgroup form's time
+// is close to linear in the row pairs.  In row pairs, a round costs least +
+// PW_IDLE of them and the workgroup form PW_IDLE before its first.  `least` is
+// measured per plan (PW_SMALL and so on); the CFL form spills more and its
+// rounds take a sixth longer.  FP32, workgroup form with 512 threads -> wave
+// form: 16 shells of 64 x 128 points (512 row pairs) 30 -> 42 us, so workgroup;
+// 32 shells 55 -> 44 us, so wave; at n = 512, 20 shells of 256 points 85 -> 90 us
+// (the second round a quarter full), 32 shells 127 -> 105, 96 shells 353 -> 311.
+// With its threads fitted to n the workgroup form stays the faster one of a
+// lone run for up to twice as many row pairs, but it takes the whole GPU where
+// the wave form leaves CUs to other runs: from the higher bounds twelve runs
+// of 32 to 86 degrees together took 103 ms, from these 100.
 constexpr long PW_IDLE = 500;
 template <class PL>
 bool physwave_pays(const Ctx& c, long least, bool cfl) {
@@ -673,26 +677,27 @@ int physwave_f32_long(Ctx& c, PwArgs<float>& a, bool cfl);
     case n: return physwave_run<R, n, r0, r1, p>(c, a, cfl, least)
 
 // Radices: the first at most one butterfly per lane, the last (points per
-// lane) 6 to 9 where the length allows, so that three vectors stay in
-// registers, with as many of the 64 lanes in use as the factors give.  Last,
-// the row pairs from which a plan beats the workgroup form (0: from one
-// shell's on, measured from 7 shells), at L = M = n / 3 with both vector
-// fields, codensity and composition.
+// lane) 6 to 9 where the length allows, with as many of the 64 lanes in use as
+// the factors give.  P = 6 holds three vectors in 256 registers; P = 8 and 9
+// spill up to 368 bytes a lane (the CFL form 204 to 648).  Last, the row pairs from which
+// a plan is no slower than the workgroup form with 512 threads (0: from one
+// shell's on, measured from 7 shells), at L = M = n / 3 with both vector fields,
+// codensity and composition.
 #define PW_SMALL(R)               \
-    PW_CASE(R, 36, 6, 1, 6, 650);      \
-    PW_CASE(R, 48, 8, 1, 6, 670);      \
-    PW_CASE(R, 54, 9, 1, 6, 560);      \
-    PW_CASE(R, 64, 8, 1, 8, 2450);      \
-    PW_CASE(R, 72, 9, 1, 8, 720);      \
-    PW_CASE(R, 96, 12, 1, 8, 1100);     \
-    PW_CASE(R, 108, 12, 1, 9, 1200);    \
-    PW_CASE(R, 128, 16, 1, 8, 2000);    \
-    PW_CASE(R, 144, 16, 1, 9, 1200);    \
-    PW_CASE(R, 162, 18, 1, 9, 900);    \
-    PW_CASE(R, 192, 8, 4, 6, 620);     \
-    PW_CASE(R, 216, 9, 3, 8, 660)
+    PW_CASE(R, 36, 6, 1, 6, 180);      \
+    PW_CASE(R, 48, 8, 1, 6, 220);      \
+    PW_CASE(R, 54, 9, 1, 6, 250);      \
+    PW_CASE(R, 64, 8, 1, 8, 500);      \
+    PW_CASE(R, 72, 9, 1, 8, 320);      \
+    PW_CASE(R, 96, 12, 1, 8, 430);     \
+    PW_CASE(R, 108, 12, 1, 9, 500);    \
+    PW_CASE(R, 128, 16, 1, 8, 850);    \
+    PW_CASE(R, 144, 16, 1, 9, 650);    \
+    PW_CASE(R, 162, 18, 1, 9, 600);    \
+    PW_CASE(R, 192, 8, 4, 6, 420);     \
+    PW_CASE(R, 216, 9, 3, 8, 500)
 #define PW_LARGE(R)               \
-    PW_CASE(R, 256, 8, 4, 8, 900);     \
+    PW_CASE(R, 256, 8, 4, 8, 600);     \
     PW_CASE(R, 288, 8, 6, 6, 0);     \
     PW_CASE(R, 324, 9, 6, 6, 0);     \
     PW_CASE(R, 384, 8, 8, 6, 0);     \
