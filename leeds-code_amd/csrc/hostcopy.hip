@@ -26,8 +26,9 @@ constexpr size_t HC_CHUNK = size_t(1) << 20;
 // directly, 189 through the chunks; new arrays 606 and 433.  Uploads find
 // their pages mapped and gain later, analysis of one field and of three: 4.7 MB
 // 253 us directly, 346 through the chunks; 18.9 MB 770 and 883 (new arrays
-// 940, 920), 28.3 MB 1140-1380 and 1302 (1410, 1340), 56.6 MB 2595 and 2448.
-constexpr size_t HC_MIN = size_t(2) << 20, HC_MIN_UP = size_t(24) << 20;
+// 940, 920), 28.3 MB 1140-1380 and 1302 (1410, 1340), 56.6 MB 2595 and 2448:
+// their callers say from where (HC_UPLOAD by default).
+constexpr size_t HC_MIN = size_t(2) << 20;
 
 int HostStage::reserve() {
     if (buf) return LSD_OK;
@@ -124,7 +125,7 @@ static bool overlap(const HostPart* parts, int np) {
 // in the stream's order; they may still read the host arrays (pinned ones, of
 // any size), and on an error copies either way may be under way.  The calling
 // entry point waits for the stream before it returns (CopyGuard).
-int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host) {
+int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host, size_t upload_min) {
     size_t total = 0, nq = 0;
     for (int k = 0; k < np; k++) {
         if (!parts[k].host) {
@@ -134,7 +135,7 @@ int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, 
         total += parts[k].bytes;
         nq += (parts[k].bytes + HC_CHUNK - 1) / HC_CHUNK;
     }
-    bool chunks = total >= (to_host ? HC_MIN : HC_MIN_UP);
+    bool chunks = total >= (to_host ? HC_MIN : upload_min);
     for (int k = 0; k < np && chunks; k++) chunks = pageable(parts[k].host);
     if (to_host && overlap(parts, np)) chunks = false;
     if (!chunks) {

@@ -58,7 +58,9 @@ struct HostPart {
     void* dev;
     size_t bytes;
 };
-int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host);
+constexpr size_t HC_UPLOAD = size_t(24) << 20;  // bytes from which uploads go through the chunks
+int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, bool to_host,
+              size_t upload_min = HC_UPLOAD);
 
 // Waits for the stream on every return of a call with host arrays but a
 // successful one (which waits itself): no copy still reads or writes the
