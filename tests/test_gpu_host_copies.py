@@ -1,7 +1,8 @@
-"""Copies to and from a caller's arrays below and above the size from which
-they go through pinned chunks, with a last chunk of one element, whole chunks
-and a rest: state fields set and read back, exactly; both directions of the
-network's forward pass against slices small enough for the plain copy."""
+"""Copies to and from a caller's arrays below and above the sizes from which
+they go through the host's loop, plain copies and pinned chunks, with whole
+chunks and a rest: state fields set and read back, exactly; both directions of
+the network's forward pass against slices small enough for the plain copy.
+(Rests of every kind, to one byte: test_host_copies.py.)"""
 import time
 
 import numpy as np
@@ -72,8 +73,9 @@ def test_network_forward(rows):
     net = Mlp(16, 32, 16)
     x = np.random.default_rng(rows).standard_normal((rows, 16)).astype(np.float32)
     y = net.forward(x)
-    for r in range(0, rows, 5000):
-        assert np.array_equal(y[r:r + 5000], net.forward(x[r:r + 5000]))
+    step = min(300, rows) if rows < 40000 else 5000
+    for r in range(0, rows, step):
+        assert np.array_equal(y[r:r + step], net.forward(x[r:r + step]))
 
 
 def test_failed_call_has_read_its_pinned_array():

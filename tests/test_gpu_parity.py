@@ -204,6 +204,28 @@ def test_one_step_large_grid():
     g.close()
 
 
+@pytest.mark.parametrize("L,M,Mp,N", [(32, 8, 4, 96), (29, 8, 4, 65), (20, 1, 1, 96), (300, 2, 1, 70), (64, 64, 1, 64),
+                                      (12, 12, 1, 7)])
+def test_energy_spectra_sizes(L, M, Mp, N):
+    # every fourth order, one order, more than one radial point a lane (N > 64),
+    # more degrees and orders than a workgroup has work-items
+    cfg = make_config(L=L, M=M, Mp=Mp, N=N, Th=(3 * L // 2 + 1) // 2 * 2, Ph=max(4, 3 * M), dt=1e-6)
+    g = Context(cfg)
+    o = O.Oracle(cfg)
+    st = seeded_state(cfg, 19, 1e-2)
+    g.set_state(st)
+    o.set_state(st)
+    for which in (0, 1):
+        E, El, Em = g.energy(which)
+        Eo, Elo, Emo = o.energy(which)
+        assert abs(E - Eo) <= 1e-12 * Eo
+        # sums of squares of about N H terms at most, every one positive
+        assert np.all(np.abs(El - Elo) <= 1e-12 * Elo) and np.all(np.abs(Em - Emo) <= 1e-12 * Emo)
+        assert np.count_nonzero(Em) == M
+    g.close()
+
+
+
 @pytest.mark.parametrize("which", [0, 1])
 def test_energy_spectra(pair, which):
     # lsd_energy against the oracle's Parseval-pinned energies
