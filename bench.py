@@ -103,11 +103,15 @@ def cpu_baseline(cfg, state, threads, ref_steps):
     return out
 
 
-def load_traffic(kernel_class):
+PHYS_KERNEL = "k_physwave"  # the physical-space pass at this workload's sizes
+
+
+def load_traffic(kernel):
+    """HBM bytes per launch of this kernel; None if they were measured on another."""
     path = os.path.join(ROOT, "profiles", "traffic.json")
     try:
         with open(path) as f:
-            return json.load(f).get(kernel_class)
+            return json.load(f).get(kernel)
     except (OSError, ValueError):
         return None
 
@@ -277,11 +281,11 @@ def main():
     achieved = per_launch / avg_s / 1e9
     roof = {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
             "frac": achieved / PEAK_HBM_GBS}
-    roof["kernel"] = "k_physwave (class %s)" % K_NAMES[dom]
+    roof["kernel"] = "%s (class %s)" % (PHYS_KERNEL, K_NAMES[dom])
     roof["algorithmic_bytes_per_launch"] = per_launch
     roof["launches"] = nl
     roof["avg_launch_ms"] = avg_s * 1e3
-    roof["traffic"] = load_traffic(K_NAMES[dom])
+    roof["traffic"] = load_traffic(PHYS_KERNEL)
 
     evals = st.evaluations / max(st.steps, 1)
     leg_flops = pc["synth"]["work"] + pc["anal"]["work"]
