@@ -30,12 +30,14 @@ constexpr size_t HC_CHUNK = size_t(1) << 20;
 // their callers say from where (HC_UPLOAD by default).
 constexpr size_t HC_MIN = size_t(2) << 20;
 
-int HostStage::reserve() {
-    if (buf) return LSD_OK;
+bool HostStage::reserve() {
+    if (buf) return true;
     for (hipEvent_t& e : ev)
-        if (!e) LSD_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    LSD_HIP(hipHostMalloc((void**)&buf, 2 * HC_THREADS * HC_CHUNK, hipHostMallocDefault));
-    return LSD_OK;
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) e = nullptr;
+    for (const hipEvent_t& e : ev)
+        if (!e) return false;
+    if (hipHostMalloc((void**)&buf, 2 * HC_THREADS * HC_CHUNK, hipHostMallocDefault) != hipSuccess) buf = nullptr;
+    return buf != nullptr;
 }
 
 void HostStage::release() {
@@ -138,6 +140,11 @@ int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, 
     bool chunks = total >= (to_host ? HC_MIN : upload_min);
     for (int k = 0; k < np && chunks; k++) chunks = pageable(parts[k].host);
     if (to_host && overlap(parts, np)) chunks = false;
+    if (chunks && !st.reserve()) {
+        // no pinned memory to be had: a plain copy needs none of it
+        (void)hipGetLastError();
+        chunks = false;
+    }
     if (!chunks) {
         for (int k = 0; k < np; k++)
             LSD_HIP(hipMemcpyAsync(to_host ? parts[k].host : parts[k].dev, to_host ? parts[k].dev : parts[k].host,
@@ -145,8 +152,6 @@ int host_copy(HostStage& st, hipStream_t stream, const HostPart* parts, int np, 
         if (to_host) LSD_HIP(hipStreamSynchronize(stream));
         return LSD_OK;
     }
-    const int rc = st.reserve();
-    if (rc) return rc;
     int device = 0;
     LSD_HIP(hipGetDevice(&device));
     hipError_t err[HC_THREADS];

@@ -50,7 +50,7 @@ void harmonics(int L, int M, int Mp, std::vector<int>& hl, std::vector<int>& hm)
 struct HostStage {
     char* buf = nullptr;
     hipEvent_t ev[8] = {};
-    int reserve();
+    bool reserve();  // false: no pinned memory or events
     void release();
 };
 struct HostPart {

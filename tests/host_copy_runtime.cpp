@@ -32,7 +32,7 @@ struct Lock {
     Lock() { in_runtime = true; }
     ~Lock() { in_runtime = false; }
 };
-int caller_delay_ms = 0, copies_ok = -1, threads_fail = 0;
+int caller_delay_ms = 0, copies_ok = -1, threads_fail = 0, no_pinned = 0;
 
 bool is_pinned(const void* p) {
     auto it = pinned.upper_bound((const char*)p);
@@ -89,6 +89,7 @@ hipError_t hipEventSynchronize(hipEvent_t e) {
     return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (no_pinned) return hipErrorOutOfMemory;
     *p = malloc(n);
     Lock lock;
     pinned[(const char*)*p] = n;
@@ -133,9 +134,10 @@ void set_error(const std::string&) {}
 extern "C" {
 // One host_copy of np parts.  pin: the host arrays are pinned.  delay_ms:
 // the calling thread waits that long at every event.  ok: hipMemcpyAsync
-// fails after so many calls (-1: never).  oom: no memory for threads.
+// fails after so many calls (-1: never).  oom: no memory for threads.  nopin:
+// no pinned memory.
 int fake_host_copy(int np, void** host, void** dev, const size_t* bytes, int to_host, int pin, int delay_ms, int ok,
-                   int oom) {
+                   int oom, int nopin) {
     lsd::HostStage st;
     lsd::HostPart parts[8];
     caller = std::this_thread::get_id();
@@ -146,13 +148,14 @@ int fake_host_copy(int np, void** host, void** dev, const size_t* bytes, int to_
         if (pin) pinned[(const char*)host[k]] = bytes[k];
     }
     threads_fail = oom;
+    no_pinned = nopin;
     int rc;
     try {
         rc = lsd::host_copy(st, nullptr, parts, np, to_host != 0);
     } catch (const std::exception&) {
         rc = -99;  // through a C entry point this would end the program
     }
-    threads_fail = 0;
+    threads_fail = no_pinned = 0;
     copies_ok = -1;
     caller_delay_ms = 0;
     st.release();

@@ -27,11 +27,12 @@ def lib(tmp_path_factory):
     return ctypes.CDLL(so)
 
 
-def copy(lib, host, dev, to_host, pin=False, delay=0, ok=-1, oom=False):
+def copy(lib, host, dev, to_host, pin=False, delay=0, ok=-1, oom=False, nopin=False):
     n = len(host)
     P, S = ctypes.c_void_p * n, ctypes.c_size_t * n
     return lib.fake_host_copy(n, P(*[a.ctypes.data for a in host]), P(*[a.ctypes.data for a in dev]),
-                              S(*[a.nbytes for a in host]), int(to_host), int(pin), delay, ok, int(oom))
+                              S(*[a.nbytes for a in host]), int(to_host), int(pin), delay, ok, int(oom),
+                              int(nopin))
 
 
 # below and above the sizes of the chunked copies (2 MiB of results, 24 MiB of
@@ -76,3 +77,23 @@ def test_no_memory_for_threads(lib, to_host):
     host, dev = (dst, src) if to_host else (src, dst)
     assert copy(lib, [host], [dev], to_host, oom=True) == 0
     assert np.array_equal(src, dst)
+
+
+@pytest.mark.parametrize("to_host", [True, False])
+def test_no_pinned_memory(lib, to_host):
+    """Without pinned memory for the chunks the copy is a plain one."""
+    src = np.random.default_rng(4).integers(0, 256, 25 * MB + 1, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    host, dev = (dst, src) if to_host else (src, dst)
+    assert copy(lib, [host], [dev], to_host, nopin=True) == 0
+    assert np.array_equal(src, dst)
+
+
+@pytest.mark.parametrize("to_host", [True, False])
+@pytest.mark.parametrize("ok", [0, 3])
+def test_failing_copy(lib, to_host, ok):
+    """A copy that the runtime refuses is reported."""
+    src = np.ones(25 * MB + 1, dtype=np.uint8)
+    dst = np.zeros_like(src)
+    host, dev = (dst, src) if to_host else (src, dst)
+    assert copy(lib, [host], [dev], to_host, ok=ok) != 0
