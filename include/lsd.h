@@ -19,6 +19,14 @@
  *
  * One context = one HIP device + one stream; all fields stay resident in
  * HBM between calls.  Contexts are not shared between host threads.
+ *
+ * Host arrays may be pageable or pinned; a call has finished with them when it
+ * returns, also with an error.  Large copies (results from 2 MiB, inputs from
+ * 24 MiB; the network's from 16 MiB) of pageable arrays go through 8 MiB of
+ * pinned memory that the context or network allocates at the first of them and
+ * keeps until it is destroyed, and start three threads for the copy.  Result
+ * arrays that share memory hold what the last of them in the argument list
+ * brings.
  */
 #ifndef LSD_H
 #define LSD_H
@@ -329,7 +337,9 @@ int lsd_sync(lsd_ctx* ctx);
  *            factors with one FP64-residual refinement sweep), 2 FP64
  *            factors in the mixed forms: register columns padded to a
  *            multiple of 16 rows for other N <= 128, else LDS-column (their
- *            default for other N) */
+ *            default for other N).  Contexts of the mixed forms with such an
+ *            N <= 128 hold seven more coll arrays for it (16 H N bytes each:
+ *            0.5 GB at L = M = 256, N = 128) */
 #define LSD_V_SYN_SCALAR 0
 #define LSD_V_SYN_VECTOR 1
 #define LSD_V_SYN_GRAD   2
@@ -379,6 +389,10 @@ int lsd_profile_end(lsd_ctx* ctx, double* total_ms, int* launches, double* work)
  * by Adam on a mean-squared-error loss.  Parameters, FP32 and contiguous:
  * W1[width][n_in] b1[width] W2[width][width] b2[width] W3[n_out][width]
  * b3[n_out].  Rows of x / y / target are contiguous, host memory.
+ * A network keeps its device buffers for the next call until it is destroyed:
+ * inputs and outputs of the largest call, activations and gradients of the
+ * largest batch, the largest training set, and the loss partials of up to 256
+ * steps (4 MiB, or one step's where they are more, there and pinned).
  * ---------------------------------------------------------------------- */
 typedef struct lsd_mlp lsd_mlp;
 int  lsd_mlp_create(int n_in, int width, int n_out, unsigned long long seed, lsd_mlp** out);

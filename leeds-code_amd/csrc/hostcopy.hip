@@ -9,8 +9,8 @@
 // array, so the page mapping and the host copies of the threads run side by
 // side with the transfers.  The chunks belong to one context or network and
 // are freed with it.  Three components to the grid and back at L = M = 64,
-// N = 64, 96 x 192 (69 MB): 5.6 -> 3.4 ms; the closure network on 57792 rows
-// of 92 values: 0.98-1.05 -> 0.96 ms, its first call 1.8 -> 1.2 ms.
+// N = 64, 96 x 192 (69 MB), in new arrays: 4.2 -> 3.4 ms; one field to the grid
+// in arrays that are kept (19 MB): 1.31 -> 0.82 ms.
 #include <cstring>
 #include <exception>
 #include <thread>

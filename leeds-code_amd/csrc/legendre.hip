@@ -20,8 +20,8 @@
 // Analysis (modules/transform.fftw3.F90:527-602, 825-949).  The forward FFT
 // leaves folded data G_p[j, c] (north+south, south-north), contracted as
 // D[k, c] = sum_j Tw[j, k] G[j, c] with the quadrature-weighted tables.  In
-// k_ana (FP32, odd Th2 and the LDS-staged variant) a workgroup takes one slot and 32 columns, stages 16-theta chunks of
-// G through LDS, and each wave contracts 16-harmonic tiles of one parity
+// k_ana (FP32, odd Th2 and the LDS-staged variant) a workgroup takes one slot
+// and 32 columns, stages 16-theta chunks of G through LDS, and each wave contracts 16-harmonic tiles of one parity
 // class against them, with the tables stored [j][h] and each slot's even-k
 // harmonics before its odd-k ones, so table reads and result writes are
 // 128-byte runs.  The FP64 form k_ana8 and the FP32 form k_ana4 (below, for
@@ -1161,7 +1161,8 @@ k_ana(AnaArgs<T> a) {
 // against 9.5 KB of operands, from L2 mostly; the barriers and single wave per SIMD of the
 // LDS-staged form left the matrix cores idle 4 cycles in 5.  L = M = 170,
 // N = 96, both vector fields: 483 -> 264 us (27 of 73 TFLOP/s), scalars 75 ->
-// 70 us; L = M = 32, N = 32: 14.6 -> 6.6 us.
+// 70 us; L = M = 32, N = 32: 14.6 -> 6.6 us.  The vector kind spills 28 bytes a
+// lane at three tiles and 256 registers.
 constexpr int A8_TP = 3;   // harmonic tiles per wave at most
 constexpr int A8_SH = 16;  // shells per wave
 constexpr int A8_NB = 2;   // operand buffers

@@ -229,8 +229,8 @@ struct Ctx {
     int n_partial_blocks = 0;          // solve blocks per field
     int solve_hb = 0;                  // harmonics per solve block
 
-    // kernel variants (LSD_V_*), see lsd_set_variant
     HostStage stage;                   // copies to and from the caller's arrays
+    // kernel variants (LSD_V_*), see lsd_set_variant
     int var[LSD_V_COUNT] = {4, 8, 8, 0, 0};
     bool ana_wide_ok = false;          // the wide-load FP32 analysis applies (even Th2)
     bool solve_direct_ok = false;      // the two-pass solves apply (N in {32, 48, 64, 96})

@@ -1,5 +1,6 @@
 // Shared declarations of the banded-solve kernels (solve.hip: columns in
-// LDS, any N; solve_direct.hip: two passes, N fixed at compile time).
+// LDS, any N; solve_direct.hip: two passes, columns of up to 128 rows in
+// registers).
 #pragma once
 
 #include "lsd_internal.h"

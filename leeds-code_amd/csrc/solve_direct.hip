@@ -383,8 +383,9 @@ __device__ __forceinline__ void load_rows(const ColRows<N, EXACT>& cr, const C* 
 }
 
 // Predictor solves: x* = X^-1 b for the right-hand sides of k_rhs_pred.  Up
-// to N = 96 at most 256 VGPRs, so two waves share each SIMD; longer columns
-// have a SIMD to themselves.
+// to N = 96 at most 256 VGPRs, so two waves share each SIMD (at 96 rows with 20
+// bytes a lane in scratch, padded columns 68); longer columns have a SIMD to
+// themselves.
 template <int N, bool EXACT>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(N <= 96 ? 2 : 1))) k_spred(DirArgs a) {
     static_assert(N % DIR_BATCH == 0, "N must be a multiple of the batch");

@@ -3,10 +3,11 @@ columns padded with identity rows to a multiple of 16, at the smallest and
 largest N, at whole multiples of 16 and one row to either side, with partial
 blocks of harmonics, against the plain form's LDS-column solves.
 
-Both forms solve in FP64 and differ in the FP32 nonlinear terms N, of which
-dt N enters the state.  dt |N| < |x| here, so the states differ by less than
-one FP32 rounding, 2^-24 = 6e-8, a step; a wrong row of a solve shows at the
-order of its value."""
+States after steps: both forms solve in FP64 and differ in the FP32 nonlinear
+terms N, of which dt N enters the state.  dt |N| < |x| here, so the states differ
+by less than one FP32 rounding, 2^-24 = 6e-8, a step; a wrong row of the predictor
+shows at the order of its value.  The corrector's changes are smaller than that
+bound in most fields: they are compared by themselves, on equal N."""
 import numpy as np
 import pytest
 
