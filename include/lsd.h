@@ -24,7 +24,8 @@
  * returns, also with an error.  Large copies (results from 2 MiB, inputs from
  * 24 MiB; the network's from 16 MiB) of pageable arrays go through 8 MiB of
  * pinned memory that the context or network allocates at the first of them and
- * keeps until it is destroyed, and start three threads for the copy.  Result
+ * keeps until it is destroyed, and start three threads for the copy; a small
+ * field's pairs take up to 1 MiB of pageable memory, kept alike.  Result
  * arrays that share memory hold what the last of them in the argument list
  * brings.
  */

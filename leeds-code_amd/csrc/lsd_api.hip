@@ -7,7 +7,6 @@
 #include <cstdlib>
 #include <cmath>
 #include <cstring>
-#include <memory>
 #include <new>
 #include <string>
 #include <vector>
@@ -571,14 +570,16 @@ static int copy_pair(Ctx& c, const double* re, const double* im, double* tmp, bo
 // over it) took reading the six fields from 42 to 25 ms at L = M = 170, N = 96
 // and from 160 to 63-80 ms at L = M = 256, N = 128; the pinned chunks of
 // host_copy then take it to 20 and 60 ms.  It costs a launch and a second
-// copy, so small fields go through the host's loop: 0.27 MB set 23 us there, 40
-// here, 0.81 MB 52 and 53; 0.27 MB read 27 and 43 (new arrays 28 and 77), 1.06
-// MB 119 and 78 (new arrays 122 and 229: nothing but the runtime maps their
-// pages), 2.1 MB, where the chunks begin, 222 and 149 (245 and 149).
-constexpr size_t SPLIT_SET = size_t(768) << 10, SPLIT_GET = size_t(2) << 20;
-static std::unique_ptr<double2[]> small_pairs(const Ctx& c, size_t split) {
+// copy, so small fields go through the host's loop: 0.27 MB set in 23 us there
+// and 40 so, 0.81 MB in 52 and 53; 0.27 MB read in 27 and 44 us, 0.90 MB in 65 and
+// 72, 1.2 MB in 117 and 85.  Its pairs stay with the context: the pages of a new
+// buffer would be mapped on every call.
+constexpr size_t SPLIT_SET = size_t(768) << 10, SPLIT_GET = size_t(1) << 20;
+static double2* small_pairs(Ctx& c, size_t split) {
     const size_t n = c.coll_elems();
-    return std::unique_ptr<double2[]>(n * sizeof(double2) < split ? new (std::nothrow) double2[n] : nullptr);
+    if (n * sizeof(double2) >= split) return nullptr;
+    if (!c.pairs) c.pairs.reset(new (std::nothrow) double2[n]);
+    return c.pairs.get();
 }
 static double* coll_staging(Ctx& c) {
     static_assert(SI_COUNT >= 1, "at least one double2 coll array");
@@ -1318,11 +1319,11 @@ int lsd_set_coll(lsd_ctx* ctx, int field, const double* re, const double* im) {
     }
     const size_t HN = c.coll_elems();
     double* tmp = lsd::coll_staging(c);
-    const auto pairs = lsd::small_pairs(c, lsd::SPLIT_SET);
+    double2* const pairs = lsd::small_pairs(c, lsd::SPLIT_SET);
     lsd::CopyGuard guard(c.stream);
     if (pairs) {
         for (size_t q = 0; q < HN; q++) pairs[q] = make_double2(re[q], im[q]);
-        LSD_HIP(hipMemcpyAsync(c.d_f[field], pairs.get(), sizeof(double2) * HN, hipMemcpyHostToDevice, c.stream));
+        LSD_HIP(hipMemcpyAsync(c.d_f[field], pairs, sizeof(double2) * HN, hipMemcpyHostToDevice, c.stream));
         LSD_HIP(hipStreamSynchronize(c.stream));
         return guard.pass(LSD_OK);
     }
@@ -1530,10 +1531,10 @@ int lsd_get_coll(lsd_ctx* ctx, int field, double* re, double* im) {
     }
     const size_t HN = c.coll_elems();
     double* tmp = lsd::coll_staging(c);
-    const auto pairs = lsd::small_pairs(c, lsd::SPLIT_GET);
+    double2* const pairs = lsd::small_pairs(c, lsd::SPLIT_GET);
     lsd::CopyGuard guard(c.stream);
     if (pairs) {
-        LSD_HIP(hipMemcpyAsync(pairs.get(), c.d_f[field], sizeof(double2) * HN, hipMemcpyDeviceToHost, c.stream));
+        LSD_HIP(hipMemcpyAsync(pairs, c.d_f[field], sizeof(double2) * HN, hipMemcpyDeviceToHost, c.stream));
         LSD_HIP(hipStreamSynchronize(c.stream));
         for (size_t q = 0; q < HN; q++) {
             re[q] = pairs[q].x;

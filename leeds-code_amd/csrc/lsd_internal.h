@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -230,6 +231,7 @@ struct Ctx {
     int solve_hb = 0;                  // harmonics per solve block
 
     HostStage stage;                   // copies to and from the caller's arrays
+    std::unique_ptr<double2[]> pairs;  // a small field on its way (below 1 MiB)
     // kernel variants (LSD_V_*), see lsd_set_variant
     int var[LSD_V_COUNT] = {4, 8, 8, 0, 0};
     bool ana_wide_ok = false;          // the wide-load FP32 analysis applies (even Th2)

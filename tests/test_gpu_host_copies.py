@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 # H = 528 (L = 32) and 4656 (L = 96) coll rows: 2 x 8 x H N bytes a field, from
 # 59 KB to 25 MB
-@pytest.mark.parametrize("L,N", [(32, 7), (32, 31), (32, 248), (32, 249), (32, 256), (96, 10),
+@pytest.mark.parametrize("L,N", [(32, 7), (32, 31), (32, 248), (32, 249), (32, 256), (32, 124), (32, 125), (96, 10),
                                  (96, 11), (96, 127), (96, 339)])
 def test_state_fields(L, N):
     cfg = make_config(L=L, M=L, N=N, dt=1e-6)
